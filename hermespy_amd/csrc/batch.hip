@@ -1272,35 +1272,123 @@ extern "C" int hpx_run_batch_drops(const hpx_link* link_host, const hpx_frame* f
 
 // ---------------------------------------------------------------- float64 single-antenna drops
 // The float64 counterpart of the fused drop for single-antenna links of up to 256 subcarriers:
-// the same counter-based streams and the same steps, every value a double, the taps evaluated
-// exactly (sum of sinusoids per sample, fading.py:293-343) instead of from Taylor blocks, and
-// the OFDM transforms as direct DFTs over a twiddle table.  One 256-thread workgroup per drop.
+// the same counter-based streams and the same steps, every value a double, the taps summed
+// exactly over their sinusoids at every sample (fading.py:293-343) instead of from Taylor blocks.
+// One 256-thread workgroup per drop, all words of the frame at once.
+//
+// Bound: float64 VALU issue.  A sinusoid at output sample n = 64 Q + 8 a + b of a path of delay d is
+// the product of three table entries, A e^{j phi} e^{j w (64 Q - d)}, e^{j 8 w a} and e^{j w b}: per
+// path (frame / 64 + 16) x terms sines and cosines instead of frame x terms, and per 8 samples and
+// term one complex product and 8 multiply-adds on table entries that LDS broadcasts.  Every phase
+// is a product w x samples near zero, which costs less rounding than a direct evaluation's
+// w x samples + phi; the products add about as much back.  The OFDM transforms are radix-4 Stockham passes over the whole
+// frame between the two signal buffers (less rounding than the direct sums they replace).  The
+// tables and the prologue's uniforms live in the receive buffer, which is empty until the channel's
+// outputs leave their registers, so four drops share a CU.  5000 drops of 64 subcarriers, 5 paths:
+// 2398 us with a sine and cosine per sample and direct sums, 478 us now.
 namespace {
 
 constexpr int kF64Threads = 256;
 constexpr int kF64MaxSubcarriers = 256;
+constexpr int kF64Run = 8;       // consecutive output samples per thread
+constexpr int kF64Block = 64;    // samples per first factor of the phase
+constexpr int kF64Round = kF64Run * kF64Threads;  // output samples per round of the workgroup
 
 struct F64Layout {
-  int off_uni, off_sos, off_tw, off_sym, off_x, off_y, off_abar, off_bits, off_red;
+  int off_sos, off_tw, off_x, off_y, off_abar, off_bits, off_red;
   int dx, frame, bits_words;
+  int term_group;  // sinusoids whose tables fit the receive buffer at once
   int64_t bytes;
 };
 
-__global__ void __launch_bounds__(kF64Threads) f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
+__device__ __forceinline__ double2 dcmul(double2 a, double2 b) {
+  return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ double2 dcfma(double2 a, double2 b, double2 c) {
+  return make_double2(fma(a.x, b.x, fma(-a.y, b.y, c.x)), fma(a.x, b.y, fma(a.y, b.x, c.y)));
+}
+__device__ __forceinline__ double2 dcadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 dcsub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+
+// One Stockham pass of radix R (4 or 2) of `rows` N-point vectors, vector v from src + v sstride to
+// dst + v dstride; with prefix > 0 the outputs k >= N - prefix are also stored N samples earlier (the
+// cyclic prefix).  tw[k] = exp(-2 pi j k / N); SIGN = +1 conjugates it.
+template <int SIGN, int R>
+__device__ __forceinline__ void f64_fft_pass(const double2* src, int sstride, double2* dst, int dstride, int rows,
+                                             int log2n, int log2ns, const double2* tw, int prefix) {
+  constexpr int kLog2R = R == 4 ? 2 : 1;
+  const int n = 1 << log2n, log2nr = log2n - kLog2R, nr = 1 << log2nr, ns = 1 << log2ns;
+  for (int item = threadIdx.x; item < rows << log2nr; item += kF64Threads) {
+    const int v = item >> log2nr, j = item & (nr - 1), pos = j & (ns - 1);
+    const int step = pos << (log2n - log2ns - kLog2R);
+    double2 a[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      a[k] = src[v * sstride + j + k * nr];
+      if (k && ns > 1) {
+        const double2 t = tw[k * step];
+        a[k] = dcmul(a[k], make_double2(t.x, SIGN < 0 ? t.y : -t.y));
+      }
+    }
+    if constexpr (R == 4) {
+      const double2 t0 = dcadd(a[0], a[2]), t1 = dcsub(a[0], a[2]), t2 = dcadd(a[1], a[3]), t3 = dcsub(a[1], a[3]);
+      const double2 t3j = SIGN < 0 ? make_double2(t3.y, -t3.x) : make_double2(-t3.y, t3.x);
+      a[0] = dcadd(t0, t2);
+      a[1] = dcadd(t1, t3j);
+      a[2] = dcsub(t0, t2);
+      a[3] = dcsub(t1, t3j);
+    } else {
+      const double2 t = a[0];
+      a[0] = dcadd(t, a[1]);
+      a[1] = dcsub(t, a[1]);
+    }
+    const int o = ((j - pos) << kLog2R) + pos;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int k = o + r * ns;
+      dst[v * dstride + k] = a[r];
+      if (k >= n - prefix) dst[v * dstride + k - n] = a[r];
+    }
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ int f64_fft_passes(int log2n) { return (log2n + 1) >> 1; }
+
+// All passes of `rows` transforms: from src (stride sstride) alternately to b (stride N) and a (stride N),
+// the last pass to last (stride lstride), which must not be the buffer it reads.
+template <int SIGN>
+__device__ __forceinline__ void f64_fft(const double2* src, int sstride, double2* a, double2* b, double2* last, int lstride,
+                                        int rows, int log2n, const double2* tw, int prefix) {
+  const int n = 1 << log2n, passes = f64_fft_passes(log2n);
+  int log2ns = 0;
+  for (int p = 0; p < passes; ++p) {
+    double2* dst = p == passes - 1 ? last : (p & 1 ? a : b);
+    const int ds = p == passes - 1 ? lstride : n, pre = p == passes - 1 ? prefix : 0;
+    if (log2n - log2ns >= 2) f64_fft_pass<SIGN, 4>(src, sstride, dst, ds, rows, log2n, log2ns, tw, pre);
+    else f64_fft_pass<SIGN, 2>(src, sstride, dst, ds, rows, log2n, log2ns, tw, pre);
+    log2ns += 2;
+    src = dst;
+    sstride = ds;
+  }
+}
+
+__global__ void __launch_bounds__(kF64Threads) __attribute__((amdgpu_waves_per_eu(4)))
+f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
   extern __shared__ __align__(16) unsigned char lds[];
-  double* uni = reinterpret_cast<double*>(lds + g.off_uni);
   double* sos = reinterpret_cast<double*>(lds + g.off_sos);
   double2* tw = reinterpret_cast<double2*>(lds + g.off_tw);    // [N] exp(-2 pi j k / N)
-  double2* sym = reinterpret_cast<double2*>(lds + g.off_sym);  // [N] one word's symbols at their bins
   double2* x = reinterpret_cast<double2*>(lds + g.off_x);      // [dx + frame] transmitted, dx leading zeros
   double2* y = reinterpret_cast<double2*>(lds + g.off_y);      // [frame] received
   double2* abar = reinterpret_cast<double2*>(lds + g.off_abar);  // [L][words] word means of the taps
   uint32_t* bits = reinterpret_cast<uint32_t*>(lds + g.off_bits);
   int* red = reinterpret_cast<int*>(lds + g.off_red);
+  double* uni = reinterpret_cast<double*>(x);       // prologue only
+  double* dir = reinterpret_cast<double*>(y);       // prologue only: [L][terms] word-mean weights
   const int tid = threadIdx.x;
   const int64_t local_drop = blockIdx.x;
   const uint32_t drop = static_cast<uint32_t>(a.first_drop + local_drop);
-  const int n = a.n, L = a.paths, period = a.n + a.cp;
+  const int n = a.n, L = a.paths, period = a.n + a.cp, terms = a.terms;
 
   // realisation uniforms, the data bits (stream HPX_STREAM_BITS, LSB first), twiddles
   for (int c = tid; 2 * c < a.nnorm; c += kF64Threads) {
@@ -1318,134 +1406,190 @@ __global__ void __launch_bounds__(kF64Threads) f64_drop_kernel(BatchArgs a, F64L
     sincospi(-2.0 * static_cast<double>(k) / static_cast<double>(n), &s, &c);
     tw[k] = make_double2(c, s);
   }
-  for (int i = tid; i < g.dx; i += kF64Threads) x[i] = make_double2(0.0, 0.0);
   if (tid == 0) red[0] = 0;
   __syncthreads();
 
-  // SoS table exactly as the fused kernel builds it (fading.py:326-342, :492-499)
+  // SoS table (fading.py:326-342, :492-499): per term the rate and A e^{j phi}, so that every later
+  // phase is a product rate x samples near zero, which rounds far less than rate x samples + phi
   {
     const int ns = a.sinusoids;
     const int o_los_ang = 100, o_nlos_ang = 100 + L, o_los_ph = 100 + L + L * ns, o_nlos_ph = 100 + 2 * L + L * ns;
     const double inv_fs = 1.0 / a.bandwidth;
-    for (int e = tid; e < L * a.terms; e += kF64Threads) {
-      const int p = e / a.terms, k = e - p * a.terms;
-      double* row = sos + 3 * e;
+    for (int e = tid; e < L * terms; e += kF64Threads) {
+      const int p = e / terms, k = e - p * terms;
+      double rate, phase, amp;
       if (k < ns) {
         const double ang = -M_PI + 2.0 * M_PI * uni[o_nlos_ang + p * ns + k];
-        row[0] = a.doppler * cos((2.0 * M_PI * (k + 1) + ang) / ns) * inv_fs;
-        row[1] = -M_PI + 2.0 * M_PI * uni[o_nlos_ph + p * ns + k];
-        row[2] = a.path_gains[L + p];
+        rate = a.doppler * cos((2.0 * M_PI * (k + 1) + ang) / ns) * inv_fs;
+        phase = -M_PI + 2.0 * M_PI * uni[o_nlos_ph + p * ns + k];
+        amp = a.path_gains[L + p];
       } else {
         const double ang = 2.0 * M_PI * uni[o_los_ang + p];
-        row[0] = a.los_doppler * cos(ang) * inv_fs;
-        row[1] = -M_PI + 2.0 * M_PI * uni[o_los_ph + p];
-        row[2] = a.path_gains[p];
+        rate = a.los_doppler * cos(ang) * inv_fs;
+        phase = -M_PI + 2.0 * M_PI * uni[o_los_ph + p];
+        amp = a.path_gains[p];
       }
+      double sn, cs;
+      sincos(phase, &sn, &cs);
+      double* row = sos + 3 * e;
+      row[0] = rate;
+      row[1] = amp * cs;
+      row[2] = amp * sn;
+      if (e < g.frame * 2) dir[e] = dirichlet_factor(rate, n);
     }
   }
   // spatial response of the single antenna pair: exp(2 pi j u_00) (fading.py:476-489)
   double2 S;
   sincospi(2.0 * uni[0], &S.y, &S.x);
   __syncthreads();
-  for (int e = tid; e < L * a.words; e += kF64Threads) {
-    const int p = e / a.words, w = e - p * a.words;
-    abar[e] = path_in_range(a, p)
-                  ? tap_mean(sos + 3 * p * a.terms, a.terms, static_cast<double>(w) * period + a.cp, n)
-                  : make_double2(0.0, 0.0);
-  }
-
-  // transmit: map, inverse DFT (unnormalised, the constellation carries sqrt(P / N)), prefix
-  for (int w = 0; w < a.words; ++w) {
-    for (int q = tid; q < n; q += kF64Threads) {
-      const int bin = subcarrier_bin(q, n, a.dc);
-      const uint32_t v = symbol_bits(bits, (w * n + q) * a.bps, a.bps);
-      const double2 p = constellation_point(a.order, 1, bits_to_label(v, a.bps));
-      sym[bin] = make_double2(p.x * a.tx_scale, p.y * a.tx_scale);
-    }
-    __syncthreads();
-    double2* xw = x + g.dx + w * period;
-    for (int k = tid; k < n; k += kF64Threads) {
-      double re = 0.0, im = 0.0;
-      for (int b = 0; b < n; ++b) {
-        const double2 t = tw[(b * k) & (n - 1)];  // exp(+2 pi j b k / N) = conj(t)
-        re += sym[b].x * t.x + sym[b].y * t.y;
-        im += sym[b].y * t.x - sym[b].x * t.y;
+  // word means (the Dirichlet closed form): four lanes per (path, word), each every fourth sinusoid
+  for (int e0 = 0; e0 < 4 * L * a.words; e0 += kF64Threads) {
+    const int e = (e0 + tid) >> 2;
+    double ar = 0.0, ai = 0.0;
+    if (e < L * a.words) {
+      const int p = e / a.words, w = e - p * a.words;
+      if (path_in_range(a, p)) {
+        const double centre = static_cast<double>(w) * period + a.cp + 0.5 * static_cast<double>(n - 1);
+        for (int k = tid & 3; k < terms; k += 4) {
+          const int i = p * terms + k;
+          const double rate = sos[3 * i];
+          const double wgt = i < g.frame * 2 ? dir[i] : dirichlet_factor(rate, n);
+          double s, c;
+          sincos(reduce_phase(rate * centre), &s, &c);
+          const double2 v = dcmul(make_double2(sos[3 * i + 1], sos[3 * i + 2]), make_double2(c, s));
+          ar = fma(wgt, v.x, ar);
+          ai = fma(wgt, v.y, ai);
+        }
       }
-      xw[a.cp + k] = make_double2(re, im);
     }
-    __syncthreads();
-    for (int i = tid; i < a.cp; i += kF64Threads) xw[i] = xw[n + i];
-    __syncthreads();
-  }
-
-  // channel: y_n = S sum_l h_l(n - d_l) x_(n - d_l) + sqrt(P / 2) (N + jN) over the frame
-  const double np = a.noise_power[local_drop];
-  const double sigma = sqrt(0.5 * np);
-  for (int i = tid; i < g.frame; i += kF64Threads) {
-    double zr = 0.0, zi = 0.0;
-    for (int p = 0; p < L; ++p) {
-      if (!path_in_range(a, p)) continue;
-      const int d = a.delays[p];
-      const int m = i - d;
-      if (m < 0) continue;
-      double hr = 0.0, hi = 0.0;
-      const double* row = sos + 3 * p * a.terms;
-      for (int k = 0; k < a.terms; ++k) {
-        if (row[3 * k + 2] == 0.0) continue;
-        double s, c;
-        sincos(reduce_phase(fma(row[3 * k], static_cast<double>(m), row[3 * k + 1])), &s, &c);
-        hr += row[3 * k + 2] * c;
-        hi += row[3 * k + 2] * s;
-      }
-      const double2 xv = x[g.dx + m];
-      zr += hr * xv.x - hi * xv.y;
-      zi += hr * xv.y + hi * xv.x;
-    }
-    // noise sample i: words (0, 1) of call i / 2 for even i, (2, 3) for odd i
-    const uint4 wn = stream_call(a.seed, drop, HPX_STREAM_NOISE, static_cast<uint32_t>(i >> 1));
-    const uint32_t w0 = (i & 1) ? wn.z : wn.x, w1 = (i & 1) ? wn.w : wn.y;
-    const double u1 = (static_cast<double>(w0 >> 8) + 0.5) * 5.9604644775390625e-08;
-    const double u2 = static_cast<double>(w1 >> 8) * 5.9604644775390625e-08;
-    const double rho = sqrt(-2.0 * log(u1));
-    double ns, nc;
-    sincospi(2.0 * u2, &ns, &nc);
-    y[i] = make_double2(S.x * zr - S.y * zi + sigma * rho * nc, S.x * zi + S.y * zr + sigma * rho * ns);
+    ar += __shfl_xor(ar, 1, 64);
+    ai += __shfl_xor(ai, 1, 64);
+    ar += __shfl_xor(ar, 2, 64);
+    ai += __shfl_xor(ai, 2, 64);
+    if (e < L * a.words && (tid & 3) == 0) abar[e] = make_double2(ar, ai);
   }
   __syncthreads();
 
-  // receive: DFT of each word's data window, ideal CSI, ZF / MMSE, demap, bit errors
+  // transmit: map every word's symbols, inverse DFTs (unnormalised, the constellation carries
+  // sqrt(P / N)), prefixes; the last pass goes to x, so an even number of passes starts there
+  {
+    double2* xd = x + g.dx;
+    const bool even = (f64_fft_passes(a.log2n) & 1) == 0;
+    double2* sym = even ? xd : y;
+    for (int e = tid; e < a.words << a.log2n; e += kF64Threads) {
+      const int w = e >> a.log2n, q = e & (n - 1);
+      const uint32_t v = symbol_bits(bits, e * a.bps, a.bps);
+      const double2 p = constellation_point(a.order, 1, bits_to_label(v, a.bps));
+      sym[(w << a.log2n) + subcarrier_bin(q, n, a.dc)] = make_double2(p.x * a.tx_scale, p.y * a.tx_scale);
+    }
+    __syncthreads();
+    f64_fft<+1>(sym, n, even ? xd : y, even ? y : xd, xd + a.cp, period, a.words, a.log2n, tw, a.cp);
+    for (int i = tid; i < g.dx; i += kF64Threads) x[i] = make_double2(0.0, 0.0);
+    __syncthreads();
+  }
+
+  // channel: y_n = S sum_l h_l(n - d_l) x_(n - d_l) + sqrt(P / 2) (N + jN) over the frame, a round of
+  // kF64Round samples at a time from the end of the frame (the tables lie at the start of y)
+  const double np = a.noise_power[local_drop];
+  const double sigma = sqrt(0.5 * np);
+  for (int r0 = (g.frame - 1) / kF64Round * kF64Round; r0 >= 0; r0 -= kF64Round) {
+    const int blocks = (min(kF64Round, g.frame - r0) + kF64Block - 1) / kF64Block;
+    const int n0 = r0 + kF64Run * tid;
+    const bool active = n0 < g.frame;
+    double2 z[kF64Run];
+#pragma unroll
+    for (int b = 0; b < kF64Run; ++b) z[b] = make_double2(0.0, 0.0);
+    for (int p = 0; p < L; ++p) {
+      if (!path_in_range(a, p)) continue;
+      const int d = a.delays[p];
+      double2 h[kF64Run];
+#pragma unroll
+      for (int b = 0; b < kF64Run; ++b) h[b] = make_double2(0.0, 0.0);
+      for (int t0 = 0; t0 < terms; t0 += g.term_group) {
+        const int tg = min(g.term_group, terms - t0);
+        // tables [tg][blocks | 8 | 8]
+        const int row = blocks + 2 * kF64Run;
+        __syncthreads();
+        for (int e = tid; e < tg * row; e += kF64Threads) {
+          const int k = e / row, c = e - k * row;
+          const double* sp = sos + 3 * (p * terms + t0 + k);
+          const int m = c < blocks ? r0 + c * kF64Block - d
+                        : c < blocks + kF64Run ? (c - blocks) * kF64Run : c - blocks - kF64Run;
+          double sn, cs;
+          sincos(reduce_phase(sp[0] * static_cast<double>(m)), &sn, &cs);
+          const double2 v = make_double2(cs, sn);
+          y[e] = c < blocks ? dcmul(make_double2(sp[1], sp[2]), v) : v;
+        }
+        __syncthreads();
+        if (active) {
+          const double2* tq = y + (n0 - r0) / kF64Block;
+          const double2* ta = y + blocks + ((n0 / kF64Run) & (kF64Block / kF64Run - 1));
+          const double2* tb = y + blocks + kF64Run;
+          for (int k = 0; k < tg; ++k) {
+            const double2 c = dcmul(tq[k * row], ta[k * row]);
+#pragma unroll
+            for (int b = 0; b < kF64Run; ++b) h[b] = dcfma(c, tb[k * row + b], h[b]);
+          }
+        }
+      }
+      if (active) {
+#pragma unroll
+        for (int b = 0; b < kF64Run; ++b) {
+          const int m = n0 + b - d;  // (x holds dx >= d zeros before the frame)
+          if (n0 + b < g.frame) z[b] = dcfma(h[b], x[g.dx + m], z[b]);
+        }
+      }
+    }
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int b = 0; b < kF64Run; b += 2) {
+        // noise sample i: words (0, 1) of call i / 2 for even i, (2, 3) for odd i
+        const uint4 wn = stream_call(a.seed, drop, HPX_STREAM_NOISE, static_cast<uint32_t>((n0 + b) >> 1));
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+          const int i = n0 + b + o;
+          if (i >= g.frame) break;
+          const uint32_t w0 = o ? wn.z : wn.x, w1 = o ? wn.w : wn.y;
+          const double u1 = (static_cast<double>(w0 >> 8) + 0.5) * 5.9604644775390625e-08;
+          const double u2 = static_cast<double>(w1 >> 8) * 5.9604644775390625e-08;
+          const double rho = sigma * sqrt(-2.0 * log(u1));
+          double ns, nc;
+          sincospi(2.0 * u2, &ns, &nc);
+          const double2 v = dcmul(S, z[b + o]);
+          y[i] = make_double2(fma(rho, nc, v.x), fma(rho, ns, v.y));
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // receive: DFTs of the words' data windows, ideal CSI, ZF / MMSE, demap, bit errors
+  const bool odd = (f64_fft_passes(a.log2n) & 1) != 0;
+  double2* spec = odd ? x : y;
+  f64_fft<-1>(y + a.cp, period, y, x, spec, n, a.words, a.log2n, tw, 0);
   const double rx_scale = 1.0 / sqrt(static_cast<double>(n));
   const double s2 = a.detector == HPX_DETECT_MMSE ? np : 0.0;
   int errors = 0;
-  for (int w = 0; w < a.words; ++w) {
-    const double2* yw = y + w * period + a.cp;
-    for (int q = tid; q < n; q += kF64Threads) {
-      const int bin = subcarrier_bin(q, n, a.dc);
-      double yr = 0.0, yi = 0.0;
-      for (int k = 0; k < n; ++k) {
-        const double2 t = tw[(bin * k) & (n - 1)];
-        yr += yw[k].x * t.x - yw[k].y * t.y;
-        yi += yw[k].x * t.y + yw[k].y * t.x;
-      }
-      yr *= rx_scale;
-      yi *= rx_scale;
-      double cr = 0.0, ci = 0.0;
-      for (int p = 0; p < L; ++p) {
-        const int d = a.delays[p];
-        if (!path_in_range(a, p) || d >= a.keep_below) continue;
-        const double2 m = abar[p * a.words + w], t = tw[(bin * d) & (n - 1)];
-        cr += m.x * t.x - m.y * t.y;
-        ci += m.x * t.y + m.y * t.x;
-      }
-      const double hr = S.x * cr - S.y * ci, hi = S.x * ci + S.y * cr;
-      const double den = hr * hr + hi * hi + s2;
-      const double gain = den > 0.0 ? 1.0 / den : 0.0;  // pinv of a zero channel is zero
-      const double xr = (hr * yr + hi * yi) * gain, xi = (hr * yi - hi * yr) * gain;
-      const uint32_t rx = demap_symbol(a.mod, xr, xi);
-      const uint32_t tx = symbol_bits(bits, (w * n + q) * a.bps, a.bps);
-      errors += __popc(tx ^ rx);
-      if (equalized) equalized[local_drop * static_cast<int64_t>(a.words) * n + w * n + q] = make_double2(xr, xi);
+  for (int e = tid; e < a.words << a.log2n; e += kF64Threads) {
+    const int w = e >> a.log2n, q = e & (n - 1);
+    const int bin = subcarrier_bin(q, n, a.dc);
+    const double2 yv = spec[(w << a.log2n) + bin];
+    const double yr = yv.x * rx_scale, yi = yv.y * rx_scale;
+    double2 c = make_double2(0.0, 0.0);
+    for (int p = 0; p < L; ++p) {
+      const int d = a.delays[p];
+      if (!path_in_range(a, p) || d >= a.keep_below) continue;
+      c = dcfma(abar[p * a.words + w], tw[(bin * d) & (n - 1)], c);
     }
+    const double hr = S.x * c.x - S.y * c.y, hi = S.x * c.y + S.y * c.x;
+    const double den = hr * hr + hi * hi + s2;
+    const double gain = den > 0.0 ? 1.0 / den : 0.0;  // pinv of a zero channel is zero
+    const double xr = (hr * yr + hi * yi) * gain, xi = (hr * yi - hi * yr) * gain;
+    const uint32_t rx = demap_symbol(a.mod, xr, xi);
+    const uint32_t tx = symbol_bits(bits, e * a.bps, a.bps);
+    errors += __popc(tx ^ rx);
+    if (equalized) equalized[local_drop * static_cast<int64_t>(a.words) * n + e] = make_double2(xr, xi);
   }
   for (int off = 32; off > 0; off >>= 1) errors += __shfl_down(errors, off, 64);
   if ((tid & 63) == 0) atomicAdd(red, errors);
@@ -1491,15 +1635,19 @@ extern "C" int hpx_run_batch_f64(const hpx_link* link_host, const int32_t* delay
     o += align16(bytes);
     return at;
   };
-  g.off_uni = take(static_cast<int64_t>(a.nnorm) * sizeof(double));
+  // the prologue's uniforms alias the transmit buffer where it is long enough, which it is for every
+  // frame but the shortest; the sinusoids' tables alias the receive buffer
+  const int64_t uni_elems = (static_cast<int64_t>(a.nnorm) + 1) / 2;  // in complex128 values
   g.off_sos = take(static_cast<int64_t>(a.paths) * a.terms * 3 * sizeof(double));
   g.off_tw = take(static_cast<int64_t>(a.n) * sizeof(double2));
-  g.off_sym = take(static_cast<int64_t>(a.n) * sizeof(double2));
-  g.off_x = take(static_cast<int64_t>(g.dx + g.frame) * sizeof(double2));
+  g.off_x = take(std::max<int64_t>(g.dx + g.frame, uni_elems) * sizeof(double2));
   g.off_y = take(static_cast<int64_t>(g.frame) * sizeof(double2));
   g.off_abar = take(static_cast<int64_t>(a.paths) * a.words * sizeof(double2));
   g.off_bits = take(static_cast<int64_t>(g.bits_words) * sizeof(uint32_t));
   g.off_red = take(16);
+  // (a frame has at least 32 samples: one term's table always fits)
+  const int round = std::min(g.frame, kF64Round);
+  g.term_group = std::max(1, round / ((round + kF64Block - 1) / kF64Block + 2 * kF64Run));
   g.bytes = o;
   if (g.bytes > kMaxLds) {
     set_error("hpx_run_batch_f64: %lld bytes of LDS per drop exceed a CU's %lld", static_cast<long long>(g.bytes),

@@ -159,6 +159,7 @@ SIGNATURES = {
                                        ctypes.POINTER(HpxSectionStats), c_vp]),
     "hpx_pilot_ls": (c_int, [c_vp, c_i64, c_int, c_int, c_i64, c_int, c_vp, c_vp, c_vp, c_vp]),
     "hpx_lmmse_apply": (c_int, [c_vp, c_int, c_i64, c_int, c_vp, c_i64, c_vp, c_int, c_vp, c_vp]),
+    "hpx_lmmse_apply_sets": (c_int, [c_vp, c_int, c_i64, c_int, c_vp, c_i64, c_int, c_vp, c_vp, c_vp, c_vp]),
     "hpx_detect_estimated": (c_int, [c_vp, c_vp, c_i64, c_int, c_int, c_int, c_int, c_vp, c_vp, c_int, c_int, c_int,
                                      c_vp, c_u64, c_i64, c_vp, c_vp, c_vp]),
     "hpx_conv1d_forward": (c_int, [c_vp, c_i64, c_int, c_int, c_int, c_vp, c_vp, c_int, c_int, c_vp, c_vp, c_vp]),

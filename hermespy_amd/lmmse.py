@@ -15,10 +15,13 @@ word duration and rho_t the time correlation of the sum-of-sinusoids taps,
 J0(omega t) (``fading.py:293-343``), averaged over the link's Doppler
 distribution.  The filters depend only on the frame, the channel statistics
 and the SNR, so they are built once on the host (float64) per SNR point and
-applied on the device as one complex GEMM per launch (``hpx_lmmse_apply``).
+applied on the device as complex float32 GEMMs, all SNR points in one launch
+(``hpx_lmmse_apply_sets``).
 """
 
 from __future__ import annotations
+
+import ctypes
 
 import numpy as np
 import torch
@@ -107,6 +110,11 @@ def lmmse_filters(cfg: LinkConfig, snr_db) -> np.ndarray:
     return out
 
 
+class RowSets(list):
+    """Device lists of LS rows per SNR point (or None), each row in at most one of them: what
+    :meth:`LMMSEChannelEstimation.rows_by_set` returns, and what one launch can serve at once."""
+
+
 class LMMSEChannelEstimation:
     """Device-resident LMMSE filters of one pilot link; estimates [num_tx][drops][num_rx][words * N]."""
 
@@ -143,7 +151,14 @@ class LMMSEChannelEstimation:
         if rows_by_set is None:
             rows_by_set = self.rows_by_set(snr_index)
         lib, st = _lib.load(), _lib.stream_handle()
-        for s, rows in enumerate(rows_by_set):
+        if isinstance(rows_by_set, RowSets) and len(rows_by_set) <= self.filters.shape[0]:
+            lists = (ctypes.c_void_p * len(rows_by_set))(*[_lib.ptr(r) for r in rows_by_set])
+            counts = (ctypes.c_int32 * len(rows_by_set))(*[0 if r is None else int(r.numel()) for r in rows_by_set])
+            _lib.check(lib.hpx_lmmse_apply_sets(_lib.ptr(ls), c.num_tx, num_drops * c.num_rx, self.num_pilots,
+                                                _lib.ptr(self.filters), e, len(rows_by_set), ctypes.addressof(lists),
+                                                ctypes.addressof(counts), _lib.ptr(out), st))
+            return out
+        for s, rows in enumerate(rows_by_set):  # lists of the caller's own may share rows: the last set wins
             if rows is None or rows.numel() == 0:
                 continue
             _lib.check(lib.hpx_lmmse_apply(_lib.ptr(ls), c.num_tx, num_drops * c.num_rx, self.num_pilots,
@@ -151,12 +166,12 @@ class LMMSEChannelEstimation:
                                            _lib.ptr(out), st))
         return out
 
-    def rows_by_set(self, snr_index: np.ndarray) -> list:
+    def rows_by_set(self, snr_index: np.ndarray) -> RowSets:
         """Device lists of the LS rows (drop * num_rx + r) of every SNR point."""
 
         snr_index = np.asarray(snr_index)
         nr = self.cfg.num_rx
-        out = []
+        out = RowSets()
         for s in range(self.snr_db.size):
             drops = np.flatnonzero(snr_index == s)
             rows = (drops[:, None] * nr + np.arange(nr)[None, :]).reshape(-1).astype(np.int32)

@@ -191,6 +191,13 @@ int hpx_pilot_ls(const hpx_c64* grid, int64_t num_drops, int num_rx, int num_tx,
 int hpx_lmmse_apply(const hpx_c64* ls, int num_tx, int64_t num_rows, int num_pilots, const hpx_c64* filter,
                     int64_t elements, const int32_t* rows, int count, hpx_c64* est, void* stream);
 
+/* hpx_lmmse_apply for num_sets filters at once, filters [num_sets][num_tx][elements][num_pilots]:
+ * set i serves the counts_host[i] rows rows_host[i] (host arrays of device pointers and counts; an
+ * empty set's pointer may be NULL).  No row may be in two sets. */
+int hpx_lmmse_apply_sets(const hpx_c64* ls, int num_tx, int64_t num_rows, int num_pilots, const hpx_c64* filters,
+                         int64_t elements, int num_sets, const int32_t* const* rows_host,
+                         const int32_t* counts_host, hpx_c64* est, void* stream);
+
 /* Detection of every data element from estimated channels est [num_tx][num_drops][num_rx][words * N]
  * and received grids grid [num_drops][num_rx][words * N] (ZF or MMSE with noise_power[d]), hard
  * demapping and errors[d] = bit errors of drop first_drop + d against its Philox bits.

@@ -1,0 +1,10 @@
+// Fused drop kernels of 1x1 links for heterogeneous classes with the alternative FFT values per thread.
+#include "hpx_drop.hpp"
+
+namespace hpx {
+
+int batch_launch_alt_1(const void* plans_dev, const hpx_uneven_class& c, hipStream_t s) {
+  return launch_multi<1, true>(static_cast<const BatchArgs*>(plans_dev), c, s);
+}
+
+}  // namespace hpx

@@ -376,14 +376,15 @@ __device__ __forceinline__ void fft_pass_fast_out(float2* data, int count, int s
 // In-place complex FFT (sign SIGN, no scaling) of `count` vectors at data + v * stride in LDS,
 // natural order in and out, with the pass table `tab` (fill_fft_pass_table) and the padded
 // intermediate layout of pad shift `shift`.  Called by every thread; ends with a barrier.
-// Vectors are transformed in groups of at most MAXV * blockDim.x / N.
-template <int SIGN, int MAXV = kFftMaxPerThread>
+// Vectors are transformed in groups of at most MAXV * blockDim.x / N.  LONG = false: the caller
+// transforms no more than 256 points, and the passes for longer vectors are left out.
+template <int SIGN, int MAXV = kFftMaxPerThread, bool LONG = true>
 __device__ __forceinline__ void lds_fft_padded(float2* data, int count, int stride, int log2n, const float2* tab,
                                                int shift = kFftPadShift) {
   static_assert(MAXV % 4 == 0, "MAXV must be a multiple of 4");
   const int group = max(1, (MAXV * static_cast<int>(blockDim.x)) >> log2n);
   const int passes = fft_num_passes(log2n);
-  const bool fast = shift == kFftPadShift && log2n >= 9;  // N >= 512: passes 0 and 1 are radix 16
+  const bool fast = LONG && shift == kFftPadShift && log2n >= 9;  // N >= 512: passes 0 and 1 are radix 16
   for (int g0 = 0; g0 < count; g0 += group) {
     const int cnt = min(group, count - g0);
     float2* base = data + g0 * stride;

@@ -236,10 +236,13 @@ __host__ __device__ __forceinline__ uint32_t demap_symbol_f32_reg(float re, floa
 }
 
 // demap_symbol of a complex constellation for float32 components (bit-identical decisions).
-__host__ __device__ inline uint32_t demap_symbol_f32(const Modulation& m, const DemapBounds* d, float re, float im) {
-  const uint32_t br = pam_decide_f32(m.pam, re, d);
-  const uint32_t bi = pam_decide_f32(m.pam, im, d);
+__host__ __device__ inline uint32_t demap_symbol_f32(int pam, const DemapBounds* d, float re, float im) {
+  const uint32_t br = pam_decide_f32(pam, re, d);
+  const uint32_t bi = pam_decide_f32(pam, im, d);
   return interleave_axis_bits(br, bi);
+}
+__host__ __device__ inline uint32_t demap_symbol_f32(const Modulation& m, const DemapBounds* d, float re, float im) {
+  return demap_symbol_f32(m.pam, d, re, im);
 }
 
 // Label (MSB first) of a symbol's bits given bit i of `bits` = i-th bit.

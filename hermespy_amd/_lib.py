@@ -113,6 +113,11 @@ class HpxMassiveWork(ctypes.Structure):
 
 
 # name -> (restype, argtypes)
+class HpxAdamTensor(ctypes.Structure):
+    _fields_ = [("param", c_vp), ("grad", c_vp), ("m1", c_vp), ("m2", c_vp), ("weight", c_vp),
+                ("weight_transposed", c_vp), ("n", c_i64), ("taps", ctypes.c_int32), ("cin", ctypes.c_int32)]
+
+
 SIGNATURES = {
     "hpx_abi_version": (c_int, []),
     "hpx_last_error": (c_int, [ctypes.c_char_p, ctypes.c_size_t]),
@@ -172,6 +177,12 @@ SIGNATURES = {
     "hpx_estimate_error": (c_int, [c_vp, c_vp, c_vp, c_i64, c_int, c_int, c_i64, c_vp, c_vp, c_vp]),
     "hpx_nmse_grad": (c_int, [c_vp, c_vp, c_vp, c_i64, c_int, c_int, c_int, c_int, c_vp, c_int, c_vp, c_vp, c_vp,
                               c_vp]),
+    "hpx_nmse_grad_bf16": (c_int, [c_vp, c_vp, c_vp, c_i64, c_int, c_int, c_int, c_int, c_vp, c_int, c_vp, c_vp, c_vp,
+                                   c_vp]),
+    "hpx_net_forward": (c_int, [c_vp, c_i64, c_vp, c_vp, c_int, c_vp, c_vp, c_vp, c_vp]),
+    "hpx_net_backward": (c_int, [c_vp, c_i64, c_int, c_vp, c_vp, c_vp, c_vp]),
+    "hpx_adam_steps": (c_int, [ctypes.POINTER(HpxAdamTensor), c_int, ctypes.c_float, ctypes.c_float, ctypes.c_float,
+                               ctypes.c_float, c_i64, c_vp]),
     "hpx_adam_step": (c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                               ctypes.c_float, c_i64, c_vp]),
     "hpx_conv1d_weight_copies": (c_int, [c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp]),

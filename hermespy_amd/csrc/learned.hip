@@ -16,6 +16,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "hpx_common.hpp"
 
@@ -397,6 +398,17 @@ __device__ __forceinline__ float2 ideal_h(const float2* csi, const float2* spati
   return cmul(spatial[(d * num_rx + r) * num_tx + t], csi[d * wn + e]);
 }
 
+// the same factor by factor: the sample's entry of S and its drop's csi
+__device__ __forceinline__ const float2* ideal_parts(const float2* csi, const float2* spatial, int64_t s, int num_drops,
+                                                     int num_rx, int num_tx, int64_t wn, float2* sp) {
+  const int64_t dr = s % (static_cast<int64_t>(num_drops) * num_rx);
+  const int t = static_cast<int>(s / (static_cast<int64_t>(num_drops) * num_rx));
+  const int64_t d = dr / num_rx;
+  const int r = static_cast<int>(dr - d * num_rx);
+  *sp = spatial[(d * num_rx + r) * num_tx + t];
+  return csi + d * wn;
+}
+
 __global__ void __launch_bounds__(256) estimate_error_kernel(const float2* __restrict__ est,
                                                              const float2* __restrict__ csi,
                                                              const float2* __restrict__ spatial, int num_drops,
@@ -438,6 +450,39 @@ __device__ __forceinline__ int64_t out_index(int64_t s, int e, int words, int n)
   const int p = q / blk, u = q - p * blk;
   return (s * kPos + p) * (2 * words * blk) + 2 * (w * blk + u);
 }
+
+// The gradient pass walks a sample's output as it lies in memory, one (re, im) pair per thread and step.
+// Threads 256 apart differ by a fixed (position, word, subcarrier) step, so the pair's place is carried along
+// instead of divided out each time, and reads of the output and writes of the gradient are whole lines:
+// 4096 samples of 224 channels 90 us, bfloat16 gradients (159 us, and 117 us for the conversion, before).
+// (The accumulation keeps the grid's order, in which the channel is read in whole lines: 89 us, 129 in this one.)
+struct PairWalk {
+  int p, w, u;  // position, word, subcarrier of the position: subcarrier blk p + u of word w
+  int dp, dw, du, blk, words;
+  __device__ __forceinline__ PairWalk(int first, int step, int words_, int n) : blk(n / kPos), words(words_) {
+    const int per = words * blk;
+    p = first / per;
+    w = (first - p * per) / blk;
+    u = first - p * per - w * blk;
+    dp = step / per;
+    dw = (step - dp * per) / blk;
+    du = step - dp * per - dw * blk;
+  }
+  __device__ __forceinline__ void next() {
+    u += du;
+    w += dw;
+    p += dp;
+    if (u >= blk) {
+      u -= blk;
+      ++w;
+    }
+    if (w >= words) {
+      w -= words;
+      ++p;
+    }
+  }
+  __device__ __forceinline__ int element(int n) const { return w * n + blk * p + u; }
+};
 
 __device__ __forceinline__ int sample_group(int64_t s, int num_drops, int num_rx, const int32_t* group) {
   const int64_t d = (s % (static_cast<int64_t>(num_drops) * num_rx)) / num_rx;
@@ -494,39 +539,78 @@ __global__ void loss_finish_kernel(int num_groups, double* __restrict__ work, do
   loss[0] = used ? l / used : 0.0;
 }
 
+// One workgroup per sample; GRAD: float, or bfloat16 (uint16_t) for the backward pass.
+template <class GRAD>
 __global__ void __launch_bounds__(256) loss_grad_kernel(const float* __restrict__ out, const float2* __restrict__ csi,
                                                         const float2* __restrict__ spatial, int num_drops, int num_rx,
                                                         int num_tx, int words, int n, const int32_t* __restrict__ group,
                                                         int num_groups, const double* __restrict__ work,
-                                                        float* __restrict__ grad) {
+                                                        GRAD* __restrict__ grad) {
+  const int64_t s = blockIdx.x;
   const int64_t wn = static_cast<int64_t>(words) * n;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t num_samples = static_cast<int64_t>(num_tx) * num_drops * num_rx;
-  if (i >= num_samples * wn) return;
-  const int64_t s = i / wn;
-  const int e = static_cast<int>(i - s * wn);
-  const float2 h = ideal_h(csi, spatial, s, e, num_drops, num_rx, num_tx, wn);
-  const int64_t o = out_index(s, e, words, n);
+  const float2* row = reinterpret_cast<const float2*>(out) + s * wn;
+  float2 sp;
+  const float2* c = ideal_parts(csi, spatial, s, num_drops, num_rx, num_tx, wn, &sp);
   const float scale = static_cast<float>(work[2 * num_groups + sample_group(s, num_drops, num_rx, group)]);
-  grad[o] = scale * (out[o] - h.x);
-  grad[o + 1] = scale * (out[o + 1] - h.y);
+  PairWalk at(threadIdx.x, blockDim.x, words, n);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < wn; i += blockDim.x, at.next()) {
+    const float2 h = cmul(sp, c[at.element(n)]);
+    const float2 v = row[i];
+    const float gr = scale * (v.x - h.x), gi = scale * (v.y - h.y);
+    if constexpr (sizeof(GRAD) == 2)
+      reinterpret_cast<uint32_t*>(grad)[s * wn + i] = f2bf(gr) | static_cast<uint32_t>(f2bf(gi)) << 16;
+    else
+      reinterpret_cast<float2*>(grad)[s * wn + i] = make_float2(gr, gi);
+  }
 }
 
 // ---------------------------------------------------------------- Adam + weight copies
 // params float32 [cout][5][cin] (+ bias [cout] separately); writes w_bf16 [cout][5][cin] and the
 // transposed, flipped copy wt_bf16 [cin][5][cout] (wt[ci][k][co] = w[co][4 - k][ci]) used by
 // the backward-data convolution.
-__global__ void __launch_bounds__(256) adam_kernel(float* __restrict__ p, const float* __restrict__ g,
-                                                   float* __restrict__ m1, float* __restrict__ m2, int64_t n, float lr,
-                                                   float b1, float b2, float eps, float c1, float c2) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__device__ __forceinline__ float adam_update(float* p, const float* g, float* m1, float* m2, int64_t i, float lr,
+                                             float b1, float b2, float eps, float c1, float c2) {
   const float gi = g[i];
   const float a = b1 * m1[i] + (1.0f - b1) * gi;
   const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
   m1[i] = a;
   m2[i] = b;
-  p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+  const float v = p[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
+  p[i] = v;
+  return v;
+}
+
+__global__ void __launch_bounds__(256) adam_kernel(float* __restrict__ p, const float* __restrict__ g,
+                                                   float* __restrict__ m1, float* __restrict__ m2, int64_t n, float lr,
+                                                   float b1, float b2, float eps, float c1, float c2) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) adam_update(p, g, m1, m2, i, lr, b1, b2, eps, c1, c2);
+}
+
+// Every parameter tensor of a network in one launch, the weights' bfloat16 copies with them (ten updates and
+// five copies of at most 72 K elements were 15 launches of 4.5 us each).
+struct AdamTensors {
+  hpx_adam_tensor t[HPX_ADAM_MAX_TENSORS];
+  int first_block[HPX_ADAM_MAX_TENSORS + 1];
+  int count;
+};
+
+__global__ void __launch_bounds__(256) adam_tensors_kernel(AdamTensors a, float lr, float b1, float b2, float eps,
+                                                           float c1, float c2) {
+  int k = 0;
+  while (k + 1 < a.count && static_cast<int>(blockIdx.x) >= a.first_block[k + 1]) ++k;
+  const hpx_adam_tensor& t = a.t[k];
+  const int64_t i = static_cast<int64_t>(static_cast<int>(blockIdx.x) - a.first_block[k]) * 256 + threadIdx.x;
+  if (i >= t.n) return;
+  const uint16_t v = f2bf(adam_update(t.param, t.grad, t.m1, t.m2, i, lr, b1, b2, eps, c1, c2));
+  if (t.weight) t.weight[i] = v;
+  if (t.weight_transposed) {
+    const int row = t.taps * t.cin;
+    const int co = static_cast<int>(i / row), rest = static_cast<int>(i - static_cast<int64_t>(co) * row);
+    const int tap = rest / t.cin, ci = rest - tap * t.cin;
+    t.weight_transposed[(static_cast<int64_t>(ci) * t.taps + (t.taps - 1 - tap)) * (t.n / row) + co] = v;
+  }
 }
 
 __global__ void __launch_bounds__(256) weight_copies_kernel(const float* __restrict__ p, int cout, int cin, int taps,
@@ -542,159 +626,411 @@ __global__ void __launch_bounds__(256) weight_copies_kernel(const float* __restr
   if (wt) wt[(static_cast<int64_t>(ci) * taps + (taps - 1 - k)) * cout + co] = v;
 }
 
-// ---------------------------------------------------------------- fused inference
-// The whole estimator for G samples per workgroup: LS at the sample's pilots (y_p / x_p), the four
-// layers and the skip convolution, with every activation in LDS (bfloat16, zero halo rows), and
-// the output written straight into the estimate grid.  Numerically the layer-by-layer path: the
-// same float32 accumulation, bias, GELU and bfloat16 rounding between layers; the 64-channel
-// layers use the 32x32x16 MFMA (8 channels per lane and step).
-constexpr int kFusedSamples = 4;  // samples per workgroup: 78 KB of LDS, two workgroups per CU
-constexpr int kS8 = 8 + 4, kS64 = 64 + 8;  // padded LDS rows
+// ---------------------------------------------------------------- fused passes over the network
+// A workgroup of four wavefronts takes 2 PT samples through the whole network with every activation in
+// LDS; a wavefront owns PT tiles of 32 positions and computes all output channels of them.  Weights
+// are the A operand of the 32x32x16 bf16 MFMA and activations the B operand, so a lane ends up
+// with four consecutive channels of one position: activations go back to LDS, and results to memory,
+// as whole 8- and 16-byte pieces.  Two channel tiles are computed together, so that one activation
+// read feeds two MFMAs and one weight read PT of them (one tile a wavefront and four samples read
+// 1 KB of LDS per MFMA, which is all the LDS bandwidth there is).  A layer is computed in place: its
+// input is read in full into accumulators before its output is written, and with PT >= 2 a
+// wavefront owns whole samples.  Rows of 64 channels are stored with their 16-byte pieces permuted by
+// row (piece ^ (row & 7)), free of bank conflicts without padding: 44 KB for four samples, three workgroups
+// per CU.  All sums keep the order of the layer-by-layer convolutions and so round to the same bfloat16.
+// 16384 samples of 224 output channels on MI355X: 647 -> 481 us (635 TFLOP/s; the matrix cores are busy
+// for 30 % of it and the VALU, with tanhf 28 of some 33 instructions per hidden value, for 50 %); eight
+// samples a workgroup 495 us, one sample two wavefronts 527 us.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4n __attribute__((ext_vector_type(4)));
+constexpr int kActElems = kPos * 64;  // a sample's activations
 
-// 8-channel input (32x32x8 steps): tap k reads row (p + (k - TAPS/2) dil) mod 64
-template <int TAPS>
-__device__ __forceinline__ void fused_tile8(const uint16_t (*in)[kPos * kS8], const uint16_t* __restrict__ w, int co,
-                                            int dil, int half, int m, int kq, floatx16 (&acc)[kFusedSamples]) {
-  const uint16_t* wrow = w + static_cast<int64_t>(co) * TAPS * 8 + 4 * kq;
-#pragma unroll 1
-  for (int k = 0; k < TAPS; ++k) {
-    const bf16x4 b = *reinterpret_cast<const bf16x4*>(wrow + k * 8);
-    const int row = (32 * half + m + (k - TAPS / 2) * dil) & (kPos - 1);
-#pragma unroll
-    for (int g = 0; g < kFusedSamples; ++g) {
-      const bf16x4 a = *reinterpret_cast<const bf16x4*>(&in[g][row * kS8 + 4 * kq]);
-      acc[g] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc[g], 0, 0, 0);
-    }
+struct NetWeights {
+  const uint16_t* w[5];  // bfloat16 [cout][taps][cin]: four layers, skip
+  const float* b[5];
+};
+
+// This lane's place in the 32x32 tiles: column (position) m, half kq of the contraction / of the rows.
+struct TileLane {
+  int wave, m, kq;
+  __device__ __forceinline__ TileLane()
+      : wave(static_cast<int>(threadIdx.x) >> 6), m(static_cast<int>(threadIdx.x) & 31), kq((static_cast<int>(threadIdx.x) >> 5) & 1) {}
+  // tile t of the wavefront's PT: sample of the group and half of its positions
+  template <int PT>
+  __device__ __forceinline__ int sample(int t) const { return (wave * PT + t) >> 1; }
+  template <int PT>
+  __device__ __forceinline__ int half(int t) const { return PT == 1 ? wave & 1 : t & 1; }
+};
+
+// Orders LDS accesses of the lanes that share a sample.
+template <int PT>
+__device__ __forceinline__ void sample_sync() {
+  if constexpr (PT == 1) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
-// 64-channel input (32x32x16 steps: lanes 0-31 take channels c0..c0+7, lanes 32-63 c0+8..c0+15)
-__device__ __forceinline__ void fused_tile64(const uint16_t (*in)[kPos * kS64], const uint16_t* __restrict__ w, int co,
-                                             int dil, int half, int m, int kq, floatx16 (&acc)[kFusedSamples]) {
-  const uint16_t* wrow = w + static_cast<int64_t>(co) * kTaps * 64 + 8 * kq;
+template <int PT, int CT>
+__device__ __forceinline__ void zero_tiles(floatx16 (&acc)[CT][PT]) {
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int t = 0; t < PT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[c][t][r] = 0.0f;
+}
+
+// Weights on their way to LDS: the workgroup loads a chunk (up to 64 output channels by 64 elements of
+// their rows, whole 128-byte lines) into registers while the chunk before it is in use, and all
+// wavefronts read their fragments from the copy in LDS, rows permuted like the activations'.  (Fragments
+// read by each wavefront from memory touch 32 lines for 1 KB: 16384 samples, eight a workgroup, 536 us so, 495 us
+// through LDS.)
+struct WeightPipe {
+  uint16_t* lds;
+  uintx4 r0, r1;
+  // rows of 16 STEPS elements
+  template <int ROWS, int STEPS>
+  __device__ __forceinline__ void fetch(const uint16_t* __restrict__ w, int64_t wrow) {
+    constexpr int kPieces = 2 * STEPS, kTotal = ROWS * kPieces;
+    static_assert(kTotal == 256 || kTotal == 512, "one or two whole pieces per thread");
+    const int row = static_cast<int>(threadIdx.x) / kPieces, c = static_cast<int>(threadIdx.x) % kPieces;
+    const uint16_t* p = w + row * wrow + 8 * c;
+    r0 = *reinterpret_cast<const uintx4*>(p);
+    if constexpr (kTotal == 512) r1 = *reinterpret_cast<const uintx4*>(p + (256 / kPieces) * wrow);
+  }
+  template <int ROWS, int STEPS>
+  __device__ __forceinline__ void commit() {
+    constexpr int kPieces = 2 * STEPS, kTotal = ROWS * kPieces;
+    const int row = static_cast<int>(threadIdx.x) / kPieces, c = static_cast<int>(threadIdx.x) % kPieces;
+    uint16_t* p = lds + (row << 6) + ((c ^ (row & 7)) << 3);
+    __syncthreads();  // the chunk before is read
+    *reinterpret_cast<uintx4*>(p) = r0;
+    if constexpr (kTotal == 512) *reinterpret_cast<uintx4*>(p + (256 / kPieces) * 64) = r1;
+    __syncthreads();
+  }
+  __device__ __forceinline__ bf16x8 fragment(int tile, int step, const TileLane& ln) const {
+    return *reinterpret_cast<const bf16x8*>(lds + ((32 * tile + ln.m) << 6) + (((2 * step + ln.kq) ^ (ln.m & 7)) << 3));
+  }
+};
+
+// acc += circular convolution of 16 STEPS input channels (w: the first tile's weights of these channels,
+// rows of `wrow` elements, taps `wtap` apart).  Its first chunk is in the pipe already; `next` fetches
+// the one that follows the last.
+template <int PT, int CT, int STEPS, class Next>
+__device__ __forceinline__ void conv_channels(const uint16_t* act, WeightPipe& pipe, const uint16_t* __restrict__ w, int64_t wrow,
+                                              int wtap, int dil, const TileLane& ln, floatx16 (&acc)[CT][PT], Next next) {
 #pragma unroll 1
   for (int k = 0; k < kTaps; ++k) {
-    const int row = (32 * half + m + (k - kTaps / 2) * dil) & (kPos - 1);
+    pipe.template commit<32 * CT, STEPS>();
+    if (k + 1 < kTaps) pipe.template fetch<32 * CT, STEPS>(w + (k + 1) * wtap, wrow);
+    else next();
+    const int row = (ln.m + (k - kTaps / 2) * dil) & (kPos - 1);  // (the other half of the positions: row ^ 32)
+    const int sw = row & 7;
 #pragma unroll
-    for (int c0 = 0; c0 < 64; c0 += 16) {
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(wrow + k * 64 + c0);
+    for (int j = 0; j < STEPS; ++j) {
+      const int piece = ((2 * j + ln.kq) ^ sw) << 3;
+      bf16x8 wv[CT];
 #pragma unroll
-      for (int g = 0; g < kFusedSamples; ++g) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&in[g][row * kS64 + 8 * kq + c0]);
-        acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[g], 0, 0, 0);
+      for (int c = 0; c < CT; ++c) wv[c] = pipe.fragment(c, j, ln);
+#pragma unroll
+      for (int t = 0; t < PT; ++t) {
+        const uint16_t* a = act + ln.template sample<PT>(t) * kActElems + ((row ^ (32 * ln.template half<PT>(t))) << 6) + piece;
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(a);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[c], v, acc[c][t], 0, 0, 0);
       }
     }
   }
 }
 
-__device__ __forceinline__ void zero_acc(floatx16 (&acc)[kFusedSamples]) {
+// The same from the 8-channel input rows: a step takes two taps (lanes 0-31 the even one, 32-63 the odd
+// one; the tap beyond the last has zero weights).  These weights come straight from memory (9 KB a tile).
+template <int PT, int CT, int TAPS>
+__device__ __forceinline__ void conv_input(const uint16_t* xs, const uint16_t* __restrict__ w, const TileLane& ln,
+                                           floatx16 (&acc)[CT][PT]) {
+  const uint16_t* wl = w + ln.m * (TAPS * 8);
+#pragma unroll 3
+  for (int j = 0; j < (TAPS + 1) / 2; ++j) {
+    const int tap = 2 * j + ln.kq;
+    bf16x8 wv[CT];
 #pragma unroll
-  for (int g = 0; g < kFusedSamples; ++g)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[g][r] = 0.0f;
-}
-
-__device__ __forceinline__ void store_hidden(const floatx16 (&acc)[kFusedSamples], const float* __restrict__ bias,
-                                             int co, int half, int kq, uint16_t (*out)[kPos * kS64]) {
-  const float bv = bias[co];
-#pragma unroll
-  for (int g = 0; g < kFusedSamples; ++g)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int p = 32 * half + (r >> 2) * 8 + kq * 4 + (r & 3);
-      out[g][p * kS64 + co] = f2bf(gelu(acc[g][r] + bv));
+    for (int c = 0; c < CT; ++c) {
+      uintx4 v = *reinterpret_cast<const uintx4*>(wl + c * 32 * (TAPS * 8) + min(tap, TAPS - 1) * 8);
+      if (tap >= TAPS) v = uintx4{0u, 0u, 0u, 0u};
+      wv[c] = __builtin_bit_cast(bf16x8, v);
     }
+    const int row = (ln.m + tap - TAPS / 2) & (kPos - 1);
+#pragma unroll
+    for (int t = 0; t < PT; ++t) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(
+          xs + (ln.template sample<PT>(t) * kPos + (row ^ (32 * ln.template half<PT>(t)))) * 8);
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[c], v, acc[c][t], 0, 0, 0);
+    }
+  }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) learned_estimate_kernel(
-    const float2* __restrict__ grid, int num_drops, int num_rx, int words, int n, const int32_t* __restrict__ pidx,
-    const float2* __restrict__ pval, int num_pilots, const double* __restrict__ noise_power, int64_t num_samples,
-    const uint16_t* __restrict__ w1, const float* __restrict__ b1, const uint16_t* __restrict__ w2,
-    const float* __restrict__ b2, const uint16_t* __restrict__ w3, const float* __restrict__ b3,
-    const uint16_t* __restrict__ w4, const float* __restrict__ b4, const uint16_t* __restrict__ wsk,
-    const float* __restrict__ bsk, int cout, float* __restrict__ est) {
-  __shared__ __align__(16) uint16_t xs[kFusedSamples][kPos * kS8];
-  __shared__ __align__(16) uint16_t a0[kFusedSamples][kPos * kS64];
-  __shared__ __align__(16) uint16_t a1[kFusedSamples][kPos * kS64];
+// f(tile t, position, first of four channels, their values) over this lane's accumulators of channel tile c
+template <int PT, int CT, class F>
+__device__ __forceinline__ void each_quad(const floatx16 (&acc)[CT][PT], const TileLane& ln, F f) {
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < PT; ++t)
+        f(t, 32 * ln.template half<PT>(t) + ln.m, 32 * c + 8 * j + 4 * ln.kq,
+          floatx4{acc[c][t][4 * j], acc[c][t][4 * j + 1], acc[c][t][4 * j + 2], acc[c][t][4 * j + 3]});
+}
+
+__device__ __forceinline__ floatx4 load4(const float* p) {
+  floatx4 v;
+  __builtin_memcpy(&v, p, sizeof(v));
+  return v;
+}
+
+// where channels co .. co + 3 of position p lie in a sample's permuted rows
+__device__ __forceinline__ int act_at(int p, int co) { return (p << 6) + (((co >> 3) ^ (p & 7)) << 3) + (co & 4); }
+
+// What a training step keeps of the forward pass: per hidden layer the pre-activations and the
+// activations (rows [sample][position][channel]), and the output.
+struct Kept {
+  float* pre[3];
+  uint16_t* act[3];
+  float* out;
+};
+
+// TRAIN: the input rows come from x and everything the backward pass needs goes to `kept`; otherwise
+// the least-squares values of the sample's pilots come from the received grid and the estimate goes
+// straight to its grid (VEC: four channels are two whole subcarriers of one word, 16-byte aligned).
+template <int PT, bool TRAIN, bool VEC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PT == 1 ? 4 : 3)))
+net_forward_kernel(const float2* __restrict__ grid, int num_drops, int num_rx, int words, int n,
+                   const int32_t* __restrict__ pidx, const float2* __restrict__ pval, int num_pilots,
+                   const double* __restrict__ noise_power, const uint16_t* __restrict__ x, int64_t num_samples,
+                   NetWeights net, int cout, float* __restrict__ est, Kept kept) {
+  constexpr int kGroup = 2 * PT;
+  __shared__ __align__(16) uint16_t act[kGroup * kActElems];
+  __shared__ __align__(16) uint16_t xs[kGroup * kPos * 8];
+  __shared__ __align__(16) uint16_t chunk[64 * 64];
+  WeightPipe pipe{chunk, uintx4{}, uintx4{}};
+  pipe.fetch<64, 4>(net.w[1], kTaps * 64);
   const int tid = threadIdx.x;
-  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kFusedSamples;
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kGroup;
   const int64_t wn = static_cast<int64_t>(words) * n;
-  const int64_t dr_count = static_cast<int64_t>(num_drops) * num_rx;
-  const int pilot_words = num_pilots / kPos;
-  // input: LS at the sample's own pilots, two channels per pilot word, the stream flag, the SNR
-  for (int i = tid; i < kFusedSamples * kPos; i += 256) {
+  for (int i = tid; i < kGroup * kPos; i += 256) {
     const int g = i / kPos, p = i - g * kPos;
     const int64_t s = s0 + g;
-    uint16_t* row = &xs[g][p * kS8];
-    if (s >= num_samples) {
-      for (int c = 0; c < 8; ++c) row[c] = 0;
-      continue;
-    }
-    const int t = static_cast<int>(s / dr_count);
-    const int64_t dr = s - t * dr_count;
-    for (int v = 0; v < pilot_words; ++v) {
-      const int j = v * kPos + p;
-      const float2 x = pval[t * num_pilots + j];
-      const float2 y = grid[dr * wn + pidx[t * num_pilots + j]];
-      const float2 h = cscale(cmulc(x, y), 1.0f / cabs2(x));
-      row[2 * v] = f2bf(h.x);
-      row[2 * v + 1] = f2bf(h.y);
-    }
-    row[2 * pilot_words] = f2bf(t ? 1.0f : -1.0f);
-    row[2 * pilot_words + 1] = f2bf(snr_feature(noise_power, dr / num_rx));
-    for (int c = 2 * pilot_words + 2; c < 8; ++c) row[c] = 0;
-  }
-  __syncthreads();
-  const int wave = tid >> 6, lane = tid & 63;
-  const int half = wave & 1;
-  const int m = lane & 31, kq = lane >> 5;
-  floatx16 acc[kFusedSamples];
-  {  // layer 1: 8 -> 64 (column tile wave / 2)
-    const int co = (wave >> 1) * 32 + m;
-    zero_acc(acc);
-    fused_tile8<kTaps>(xs, w1, co, kDil1, half, m, kq, acc);
-    store_hidden(acc, b1, co, half, kq, a0);
-  }
-  __syncthreads();
-  {
-    const int co = (wave >> 1) * 32 + m;
-    zero_acc(acc);
-    fused_tile64(a0, w2, co, kDil2, half, m, kq, acc);
-    store_hidden(acc, b2, co, half, kq, a1);
-  }
-  __syncthreads();
-  {
-    const int co = (wave >> 1) * 32 + m;
-    zero_acc(acc);
-    fused_tile64(a1, w3, co, kDil3, half, m, kq, acc);
-    store_hidden(acc, b3, co, half, kq, a0);
-  }
-  __syncthreads();
-  // last layer + skip convolution straight into the estimate grid:
-  // channel co = 2 (w B + u) + {re, im} of position p -> est[s][w][B p + u]
-  const int blk = n / kPos;
-  for (int ct = wave >> 1; ct < cout / 32; ct += 2) {
-    const int co = ct * 32 + m;
-    zero_acc(acc);
-    fused_tile64(a0, w4, co, kDil4, half, m, kq, acc);
-    floatx16 sk[kFusedSamples];
-    zero_acc(sk);
-    fused_tile8<kSkipTaps>(xs, wsk, co, 1, half, m, kq, sk);
-    const float bv = b4[co], bs = bsk[co];
-    const int c2 = co >> 1, reim = co & 1;
-    const int w = c2 / blk, u = c2 - w * blk;
+    uintx4 row = uintx4{0u, 0u, 0u, 0u};
+    if (s < num_samples) {
+      if constexpr (TRAIN) {
+        row = *reinterpret_cast<const uintx4*>(x + (s * kPos + p) * 8);
+      } else {
+        // LS at the sample's own pilots, two channels per pilot word, the stream flag, the SNR
+        const int64_t dr_count = static_cast<int64_t>(num_drops) * num_rx;
+        const int pilot_words = num_pilots / kPos;
+        const int t = static_cast<int>(s / dr_count);
+        const int64_t dr = s - t * dr_count;
+        uint32_t pair[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int g = 0; g < kFusedSamples; ++g) {
-      const int64_t s = s0 + g;
-      if (s >= num_samples) continue;
+        for (int v = 0; v < 3; ++v) {
+          if (v >= pilot_words) break;
+          const int j = v * kPos + p;
+          const float2 px = pval[t * num_pilots + j];
+          const float2 y = grid[dr * wn + pidx[t * num_pilots + j]];
+          // (the products in this order: the value decides which bfloat16 neighbour it rounds to)
+          const float2 c = make_float2(fmaf(px.x, y.x, px.y * y.y), fmaf(-px.y, y.x, px.x * y.y));
+          const float2 h = cscale(c, 1.0f / cabs2(px));
+          pair[v] = f2bf(h.x) | static_cast<uint32_t>(f2bf(h.y)) << 16;
+        }
+        const uint32_t last = f2bf(t ? 1.0f : -1.0f) | static_cast<uint32_t>(f2bf(snr_feature(noise_power, dr / num_rx))) << 16;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int p = 32 * half + (r >> 2) * 8 + kq * 4 + (r & 3);
-        est[2 * (s * wn + static_cast<int64_t>(w) * n + blk * p + u) + reim] = (acc[g][r] + bv) + (sk[g][r] + bs);
+        for (int v = 0; v < 4; ++v) row[v] = v == pilot_words ? last : pair[v];
       }
     }
+    *reinterpret_cast<uintx4*>(xs + i * 8) = row;
   }
+  __syncthreads();
+  const TileLane ln;
+  auto hidden = [&](int layer, const floatx16 (&acc)[2][PT]) __attribute__((always_inline)) {
+    each_quad<PT, 2>(acc, ln, [&](int t, int p, int co, floatx4 v) __attribute__((always_inline)) {
+      v += load4(net.b[layer] + co);
+      bf16x4n h;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) h[i] = static_cast<__bf16>(gelu(v[i]));
+      const int g = ln.template sample<PT>(t);
+      *reinterpret_cast<bf16x4n*>(act + g * kActElems + act_at(p, co)) = h;
+      if constexpr (TRAIN) {
+        if (s0 + g < num_samples) {
+          const int64_t o = ((s0 + g) * kPos + p) * 64 + co;
+          *reinterpret_cast<floatx4*>(kept.pre[layer] + o) = v;
+          *reinterpret_cast<bf16x4n*>(kept.act[layer] + o) = h;
+        }
+      }
+    });
+    sample_sync<PT>();
+  };
+  {
+    floatx16 acc[2][PT];
+    zero_tiles<PT, 2>(acc);
+    static_assert(kDil1 == 1, "");
+    conv_input<PT, 2, kTaps>(xs, net.w[0], ln, acc);
+    hidden(0, acc);
+    zero_tiles<PT, 2>(acc);
+    conv_channels<PT, 2, 4>(act, pipe, net.w[1], kTaps * 64, 64, kDil2, ln, acc,
+                            [&]() __attribute__((always_inline)) { pipe.fetch<64, 4>(net.w[2], kTaps * 64); });
+    sample_sync<PT>();
+    hidden(1, acc);
+    zero_tiles<PT, 2>(acc);
+    conv_channels<PT, 2, 4>(act, pipe, net.w[2], kTaps * 64, 64, kDil3, ln, acc, [&]() __attribute__((always_inline)) {
+      if (cout >= 64) pipe.fetch<64, 4>(net.w[3], kTaps * 64);
+      else pipe.fetch<32, 4>(net.w[3], kTaps * 64);
+    });
+    sample_sync<PT>();
+    hidden(2, acc);
+  }
+  // last layer, and the skip convolution a channel tile at a time
+  const int blk = n / kPos;
+  auto last = [&](auto tiles, int ct) __attribute__((always_inline)) {
+    constexpr int CT = decltype(tiles)::value;
+    floatx16 acc[CT][PT];
+    zero_tiles<PT, CT>(acc);
+    const uint16_t* w4 = net.w[3] + static_cast<int64_t>(ct) * 32 * kTaps * 64;
+    conv_channels<PT, CT, 4>(act, pipe, w4, kTaps * 64, 64, kDil4, ln, acc, [&]() __attribute__((always_inline)) {  // (then the next tiles, if there are any)
+      const uint16_t* after = w4 + 32 * CT * kTaps * 64;
+      if (ct + CT + 1 < cout / 32) pipe.fetch<64, 4>(after, kTaps * 64);
+      else if (ct + CT < cout / 32) pipe.fetch<32, 4>(after, kTaps * 64);
+    });
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      floatx16 sk[1][PT];
+      zero_tiles<PT, 1>(sk);
+      conv_input<PT, 1, kSkipTaps>(xs, net.w[4] + static_cast<int64_t>(ct + c) * 32 * kSkipTaps * 8, ln, sk);
+      each_quad<PT, 1>(sk, ln, [&](int t, int p, int cc, floatx4 skip) __attribute__((always_inline)) {
+        const int64_t s = s0 + ln.template sample<PT>(t);
+        const int co = 32 * (ct + c) + cc, j = (cc >> 3);
+        const floatx4 main = floatx4{acc[c][t][4 * j], acc[c][t][4 * j + 1], acc[c][t][4 * j + 2], acc[c][t][4 * j + 3]};
+        const floatx4 v = (main + load4(net.b[3] + co)) + (skip + load4(net.b[4] + co));
+        if (s >= num_samples) return;
+        if constexpr (TRAIN) {
+          *reinterpret_cast<floatx4*>(kept.out + (s * kPos + p) * cout + co) = v;
+        } else {
+          // channel 2 (w B + u) + {re, im} of position p -> est[s][w][B p + u]
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int c2 = (co >> 1) + h;
+            const int w = c2 / blk, u = c2 - w * blk;
+            float* e = est + 2 * (s * wn + static_cast<int64_t>(w) * n + blk * p + u);
+            if constexpr (VEC) {
+              *reinterpret_cast<floatx4*>(e) = v;
+              break;
+            } else {
+              *reinterpret_cast<float2*>(e) = make_float2(v[2 * h], v[2 * h + 1]);
+            }
+          }
+        }
+      });
+    }
+  };
+  int ct = 0;
+#pragma unroll 1
+  for (; ct + 1 < cout / 32; ct += 2) last(std::integral_constant<int, 2>{}, ct);
+  if (ct < cout / 32) last(std::integral_constant<int, 1>{}, ct);
 }
+
+// Backward through the data: dz of the output rows [sample][position][224] -> dz of the three hidden
+// layers' pre-activations, each the transposed convolution (flipped weights [cin][taps][cout]) times
+// GELU's derivative, rounded to bfloat16 for the next one and for the weight gradients.  The sums run
+// over taps, then channels, as the layer-by-layer convolutions' do, so every value is theirs: the output
+// rows of a sample lie in LDS whole (rows of 464 bytes, free of bank conflicts), which leaves room for
+// two samples a workgroup and two workgroups a CU.
+struct Gradients {
+  const uint16_t* wt[3];  // transposed weights of layers 2, 3, 4
+  const float* pre[3];
+  uint16_t* dz[3];
+};
+constexpr int kOutChannels = 224, kOutRow = kOutChannels + 8;
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+net_backward_kernel(const uint16_t* __restrict__ dz_out, int64_t num_samples, Gradients net) {
+  constexpr int kGroup = 2, kChunks = (kOutChannels + 63) / 64;
+  __shared__ __align__(16) uint16_t rows[kGroup * kPos * kOutRow];
+  __shared__ __align__(16) uint16_t chunk[64 * 64];
+  uint16_t* act = rows;  // the hidden rows take the output rows' place
+  WeightPipe pipe{chunk, uintx4{}, uintx4{}};
+  constexpr int64_t wrow = kTaps * kOutChannels;
+  pipe.fetch<64, 4>(net.wt[2], wrow);
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kGroup;
+  constexpr int kPieces = kOutChannels / 8;
+#pragma unroll 7
+  for (int i = threadIdx.x; i < kGroup * kPos * kPieces; i += 256) {
+    const int row = i / kPieces, c = i - row * kPieces;  // (row: sample and position)
+    const int64_t s = min(s0 + (row >> 6), num_samples - 1);
+    *reinterpret_cast<uintx4*>(rows + row * kOutRow + 8 * c) =
+        *reinterpret_cast<const uintx4*>(dz_out + (s * kPos + (row & 63)) * kOutChannels + 8 * c);
+  }
+  const TileLane ln;
+  const int g = ln.sample<1>(0), half = ln.half<1>(0);
+  floatx16 acc[2][1];
+  zero_tiles<1, 2>(acc);
+  auto steps = [&](const uint16_t* a, auto count) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < decltype(count)::value; ++j) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(a + 16 * j);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        acc[c][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pipe.fragment(c, j, ln), v, acc[c][0], 0, 0, 0);
+    }
+  };
+  static_assert(kOutChannels % 64 == 32, "whole chunks and a half one");
+#pragma unroll 1
+  for (int k = 0; k < kTaps; ++k) {
+    const uint16_t* w = net.wt[2] + k * kOutChannels;
+    const int row = ((ln.m + (k - kTaps / 2) * kDil4) & (kPos - 1)) ^ (32 * half);
+    const uint16_t* a = rows + (g * kPos + row) * kOutRow + 8 * ln.kq;
+#pragma unroll
+    for (int q = 0; q + 1 < kChunks; ++q) {
+      pipe.commit<64, 4>();
+      if (q + 2 < kChunks) pipe.fetch<64, 4>(w + 64 * (q + 1), wrow);
+      else pipe.fetch<64, 2>(w + 64 * (q + 1), wrow);
+      steps(a + 64 * q, std::integral_constant<int, 4>{});
+    }
+    pipe.commit<64, 2>();
+    if (k + 1 < kTaps) pipe.fetch<64, 4>(w + kOutChannels, wrow);
+    else pipe.fetch<64, 4>(net.wt[1], kTaps * 64);
+    steps(a + 64 * (kChunks - 1), std::integral_constant<int, 2>{});
+  }
+  __syncthreads();
+  auto gradient = [&](int layer) __attribute__((always_inline)) {
+    each_quad<1, 2>(acc, ln, [&](int, int p, int co, floatx4 v) __attribute__((always_inline)) {
+      const int64_t o = (min(s0 + g, num_samples - 1) * kPos + p) * 64 + co;
+      const floatx4 pre = *reinterpret_cast<const floatx4*>(net.pre[layer] + o);
+      bf16x4n h;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) h[i] = static_cast<__bf16>(v[i] * gelu_grad(pre[i]));
+      if (layer > 0) *reinterpret_cast<bf16x4n*>(act + g * kActElems + act_at(p, co)) = h;
+      if (s0 + g < num_samples) *reinterpret_cast<bf16x4n*>(net.dz[layer] + o) = h;
+    });
+    __syncthreads();
+  };
+  gradient(2);
+  zero_tiles<1, 2>(acc);
+  conv_channels<1, 2, 4>(act, pipe, net.wt[1], kTaps * 64, 64, kDil3, ln, acc,
+                         [&]() __attribute__((always_inline)) { pipe.fetch<64, 4>(net.wt[0], kTaps * 64); });
+  __syncthreads();
+  gradient(1);
+  zero_tiles<1, 2>(acc);
+  conv_channels<1, 2, 4>(act, pipe, net.wt[0], kTaps * 64, 64, kDil2, ln, acc, [] {});
+  gradient(0);
+}
+
+// Tiles per wavefront: two (four samples a workgroup) where that still leaves two workgroups for each of the
+// 256 CUs, else one: 2044 samples 80 us with one, 2080 samples 91 us with two (88 and 145 us before), one drop
+// of four samples 38 us (58).
+int fused_tiles(int64_t samples) { return samples >= 4 * 512 ? 2 : 1; }
 
 unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
@@ -827,27 +1163,131 @@ extern "C" int hpx_estimate_error(const hpx_c64* est, const hpx_c64* csi, const 
   return check_launch("hpx_estimate_error");
 }
 
-extern "C" int hpx_nmse_grad(const float* out, const hpx_c64* csi, const hpx_c64* spatial, int64_t num_drops,
-                             int num_rx, int num_tx, int words, int num_subcarriers, const int32_t* group,
-                             int num_groups, double* work, float* grad, double* loss, void* stream) {
+namespace {
+
+template <class GRAD>
+int nmse_grad(const char* name, const float* out, const hpx_c64* csi, const hpx_c64* spatial, int64_t num_drops, int num_rx,
+              int num_tx, int words, int num_subcarriers, const int32_t* group, int num_groups, double* work, GRAD* grad,
+              double* loss, void* stream) {
   HPX_REQUIRE(num_drops >= 1 && num_drops <= 0x7fffffff && num_rx >= 1 && num_tx >= 1 && words >= 1 &&
-                  num_subcarriers % kPos == 0 && num_groups >= 1 && (group || num_groups == 1),
-              "hpx_nmse_grad: invalid sizes");
-  HPX_REQUIRE(out && csi && spatial && work && grad && loss, "hpx_nmse_grad: null pointer");
-  const int64_t wn = static_cast<int64_t>(words) * num_subcarriers;
+                  num_subcarriers >= kPos && num_subcarriers % kPos == 0 && num_groups >= 1 && (group || num_groups == 1),
+              "%s: invalid sizes", name);
+  HPX_REQUIRE(out && csi && spatial && work && grad && loss, "%s: null pointer", name);
   const int64_t samples = static_cast<int64_t>(num_tx) * num_drops * num_rx;
-  HPX_REQUIRE(samples <= 0x7fffffff, "hpx_nmse_grad: too many samples");
+  HPX_REQUIRE(samples <= 0x7fffffff, "%s: too many samples", name);
   const hipStream_t s = as_stream(stream);
   const auto* c = reinterpret_cast<const float2*>(csi);
   const auto* sp = reinterpret_cast<const float2*>(spatial);
   const int nd = static_cast<int>(num_drops);
+  const dim3 g(static_cast<unsigned>(samples));
   // work[0 .. 2 num_groups) must be zero on entry
-  hipLaunchKernelGGL(loss_accumulate_kernel, dim3(static_cast<unsigned>(samples)), dim3(256), 0, s, out, c, sp, nd,
-                     num_rx, num_tx, words, num_subcarriers, group, num_groups, work);
+  hipLaunchKernelGGL(loss_accumulate_kernel, g, dim3(256), 0, s, out, c, sp, nd, num_rx, num_tx, words, num_subcarriers,
+                     group, num_groups, work);
   hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(64), 0, s, num_groups, work, loss);
-  hipLaunchKernelGGL(loss_grad_kernel, dim3(blocks_for(samples * wn)), dim3(256), 0, s, out, c, sp, nd, num_rx,
-                     num_tx, words, num_subcarriers, group, num_groups, work, grad);
-  return check_launch("hpx_nmse_grad");
+  hipLaunchKernelGGL((loss_grad_kernel<GRAD>), g, dim3(256), 0, s, out, c, sp, nd, num_rx, num_tx, words, num_subcarriers,
+                     group, num_groups, work, grad);
+  return check_launch(name);
+}
+
+}  // namespace
+
+extern "C" int hpx_nmse_grad(const float* out, const hpx_c64* csi, const hpx_c64* spatial, int64_t num_drops,
+                             int num_rx, int num_tx, int words, int num_subcarriers, const int32_t* group,
+                             int num_groups, double* work, float* grad, double* loss, void* stream) {
+  return nmse_grad("hpx_nmse_grad", out, csi, spatial, num_drops, num_rx, num_tx, words, num_subcarriers, group,
+                   num_groups, work, grad, loss, stream);
+}
+
+extern "C" int hpx_nmse_grad_bf16(const float* out, const hpx_c64* csi, const hpx_c64* spatial, int64_t num_drops,
+                                  int num_rx, int num_tx, int words, int num_subcarriers, const int32_t* group,
+                                  int num_groups, double* work, uint16_t* grad, double* loss, void* stream) {
+  return nmse_grad("hpx_nmse_grad_bf16", out, csi, spatial, num_drops, num_rx, num_tx, words, num_subcarriers, group,
+                   num_groups, work, grad, loss, stream);
+}
+
+extern "C" int hpx_net_forward(const uint16_t* x, int64_t num_samples, const uint16_t* const* weights,
+                               const float* const* biases, int cout, float* const* pre, uint16_t* const* act, float* out,
+                               void* stream) {
+  HPX_REQUIRE(num_samples >= 0 && num_samples <= 0x7fffffff, "hpx_net_forward: invalid sample count");
+  HPX_REQUIRE(cout >= 32 && cout % 32 == 0, "hpx_net_forward: cout must be a multiple of 32 (got %d)", cout);
+  if (num_samples == 0) return HPX_OK;
+  HPX_REQUIRE(x && weights && biases && pre && act && out, "hpx_net_forward: null pointer");
+  NetWeights net;
+  Kept kept;
+  kept.out = out;
+  uintptr_t all = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out);
+  for (int i = 0; i < 5; ++i) {
+    HPX_REQUIRE(weights[i] && biases[i], "hpx_net_forward: null layer %d", i);
+    net.w[i] = weights[i];
+    net.b[i] = biases[i];
+  }
+  for (int i = 0; i < 3; ++i) {
+    HPX_REQUIRE(pre[i] && act[i], "hpx_net_forward: null layer %d", i);
+    kept.pre[i] = pre[i];
+    kept.act[i] = act[i];
+    all |= reinterpret_cast<uintptr_t>(pre[i]) | reinterpret_cast<uintptr_t>(act[i]);
+  }
+  HPX_REQUIRE((all & 15u) == 0, "hpx_net_forward: arrays must be 16-byte aligned");
+  const int pt = fused_tiles(num_samples);
+  const dim3 g(static_cast<unsigned>((num_samples + 2 * pt - 1) / (2 * pt)));
+#define HPX_FORWARD(PT)                                                                                                  \
+  hipLaunchKernelGGL((net_forward_kernel<PT, true, true>), g, dim3(256), 0, as_stream(stream),                          \
+                     static_cast<const float2*>(nullptr), 0, 0, 0, 0, static_cast<const int32_t*>(nullptr),             \
+                     static_cast<const float2*>(nullptr), 0, static_cast<const double*>(nullptr), x, num_samples, net,  \
+                     cout, static_cast<float*>(nullptr), kept)
+  if (pt == 2) HPX_FORWARD(2);
+  else HPX_FORWARD(1);
+#undef HPX_FORWARD
+  return check_launch("hpx_net_forward");
+}
+
+extern "C" int hpx_net_backward(const uint16_t* dz_out, int64_t num_samples, int cout, const uint16_t* const* weights_transposed,
+                                const float* const* pre, uint16_t* const* dz, void* stream) {
+  HPX_REQUIRE(num_samples >= 0 && num_samples <= 0x7fffffff, "hpx_net_backward: invalid sample count");
+  if (cout != kOutChannels) {  // (the shape the layer-by-layer backward convolution has)
+    set_error("hpx_net_backward: cout %d not instantiated (224)", cout);
+    return HPX_ERR_UNSUPPORTED;
+  }
+  if (num_samples == 0) return HPX_OK;
+  HPX_REQUIRE(dz_out && weights_transposed && pre && dz, "hpx_net_backward: null pointer");
+  Gradients net;
+  uintptr_t all = reinterpret_cast<uintptr_t>(dz_out);
+  for (int i = 0; i < 3; ++i) {
+    HPX_REQUIRE(weights_transposed[i] && pre[i] && dz[i], "hpx_net_backward: null layer %d", i);
+    net.wt[i] = weights_transposed[i];
+    net.pre[i] = pre[i];
+    net.dz[i] = dz[i];
+    all |= reinterpret_cast<uintptr_t>(net.wt[i]) | reinterpret_cast<uintptr_t>(pre[i]) | reinterpret_cast<uintptr_t>(dz[i]);
+  }
+  HPX_REQUIRE((all & 15u) == 0, "hpx_net_backward: arrays must be 16-byte aligned");
+  hipLaunchKernelGGL(net_backward_kernel, dim3(static_cast<unsigned>((num_samples + 1) / 2)), dim3(256), 0,
+                     as_stream(stream), dz_out, num_samples, net);
+  return check_launch("hpx_net_backward");
+}
+
+extern "C" int hpx_adam_steps(const hpx_adam_tensor* tensors, int count, float lr, float beta1, float beta2, float eps,
+                              int64_t step, void* stream) {
+  HPX_REQUIRE(count >= 0 && count <= HPX_ADAM_MAX_TENSORS && step >= 1, "hpx_adam_steps: invalid arguments");
+  AdamTensors a{};
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    const hpx_adam_tensor& t = tensors[i];
+    HPX_REQUIRE(t.n >= 0 && (t.n == 0 || (t.param && t.grad && t.m1 && t.m2)), "hpx_adam_steps: invalid tensor %d", i);
+    HPX_REQUIRE(!t.weight_transposed || (t.cin >= 1 && t.taps >= 1 && t.n % (static_cast<int64_t>(t.cin) * t.taps) == 0),
+                "hpx_adam_steps: tensor %d is not [cout][taps][cin]", i);
+    a.t[i] = t;
+    a.first_block[i] = static_cast<int>(blocks);
+    blocks += (t.n + 255) / 256;
+    HPX_REQUIRE(blocks <= 0x7fffffff, "hpx_adam_steps: too many parameters");
+  }
+  a.count = count;
+  a.first_block[count] = static_cast<int>(blocks);
+  if (blocks == 0) return HPX_OK;
+  const float c1 = static_cast<float>(1.0 - pow(static_cast<double>(beta1), static_cast<double>(step)));
+  const float c2 = static_cast<float>(1.0 - pow(static_cast<double>(beta2), static_cast<double>(step)));
+  hipLaunchKernelGGL(adam_tensors_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream), a, lr, beta1,
+                     beta2, eps, c1, c2);
+  return check_launch("hpx_adam_steps");
 }
 
 extern "C" int hpx_adam_step(float* param, const float* grad, float* m1, float* m2, int64_t n, float lr, float beta1,
@@ -887,12 +1327,28 @@ extern "C" int hpx_learned_estimate(const hpx_c64* grid, int64_t num_drops, int 
   if (samples == 0) return HPX_OK;
   HPX_REQUIRE(grid && pilot_index && pilot_values && weights && biases && est, "hpx_learned_estimate: null pointer");
   for (int i = 0; i < 5; ++i) HPX_REQUIRE(weights[i] && biases[i], "hpx_learned_estimate: null layer %d", i);
-  const int64_t blocks = (samples + kFusedSamples - 1) / kFusedSamples;
+  const int pt = fused_tiles(samples);
+  const int64_t blocks = (samples + 2 * pt - 1) / (2 * pt);
   HPX_REQUIRE(blocks <= 0x7fffffff, "hpx_learned_estimate: too many samples");
-  hipLaunchKernelGGL(learned_estimate_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream),
-                     reinterpret_cast<const float2*>(grid), static_cast<int>(num_drops), num_rx, words,
-                     num_subcarriers, pilot_index, reinterpret_cast<const float2*>(pilot_values), num_pilots, noise_power,
-                     samples, weights[0], biases[0], weights[1], biases[1], weights[2], biases[2], weights[3], biases[3],
-                     weights[4], biases[4], cout, reinterpret_cast<float*>(est));
+  NetWeights net;
+  for (int i = 0; i < 5; ++i) {
+    net.w[i] = weights[i];
+    net.b[i] = biases[i];
+  }
+  const bool vec = (num_subcarriers / kPos) % 2 == 0 && (reinterpret_cast<uintptr_t>(est) & 15u) == 0;
+#define HPX_ESTIMATE(PT, VEC)                                                                                          \
+  hipLaunchKernelGGL((net_forward_kernel<PT, false, VEC>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0,          \
+                     as_stream(stream), reinterpret_cast<const float2*>(grid), static_cast<int>(num_drops), num_rx,    \
+                     words, num_subcarriers, pilot_index, reinterpret_cast<const float2*>(pilot_values), num_pilots,   \
+                     noise_power, static_cast<const uint16_t*>(nullptr), samples, net, cout,                           \
+                     reinterpret_cast<float*>(est), Kept{})
+  if (vec) {
+    if (pt == 2) HPX_ESTIMATE(2, true);
+    else HPX_ESTIMATE(1, true);
+  } else {
+    if (pt == 2) HPX_ESTIMATE(2, false);
+    else HPX_ESTIMATE(1, false);
+  }
+#undef HPX_ESTIMATE
   return check_launch("hpx_learned_estimate");
 }

@@ -23,6 +23,7 @@ of :mod:`hermespy_amd.lmmse` is its fallback and the baseline its NMSE is measur
 
 from __future__ import annotations
 
+import ctypes
 import math
 import time
 from pathlib import Path
@@ -154,8 +155,6 @@ class ConvNetEstimator:
         in one launch (``hpx_learned_estimate``: pilot LS, the network and the skip path with the
         activations in LDS)."""
 
-        import ctypes
-
         c = self.cfg
         drops = grid.shape[0]
         if out is None:
@@ -198,6 +197,12 @@ class ConvNetEstimator:
         if params[-1][0].shape[1] != SKIP_TAPS:
             raise ValueError(f"{path}: skip convolution with {params[-1][0].shape[1]} taps, expected {SKIP_TAPS}")
         return cls(cfg, params, device)
+
+
+def _pointers(tensors) -> ctypes.Array:
+    """Host array of the tensors' device addresses."""
+
+    return (ctypes.c_void_p * len(tensors))(*[_lib.ptr(t) for t in tensors])
 
 
 class Trainer:
@@ -259,6 +264,19 @@ class Trainer:
                                             _lib.ptr(ls), _lib.stream_handle()))
         return ls
 
+    def _forward(self, x: torch.Tensor):
+        """Network output, and the hidden layers' pre-activations and activations, of input rows x."""
+
+        net, s = self.net, x.shape[0]
+        cout = net.shapes[-1][1]
+        out = torch.empty((s, POSITIONS, cout), dtype=torch.float32, device=net.device)
+        pre = [torch.empty((s, POSITIONS, n), dtype=torch.float32, device=net.device) for _, n, _ in net.shapes[:-1]]
+        act = [torch.empty((s, POSITIONS, n), dtype=torch.bfloat16, device=net.device) for _, n, _ in net.shapes[:-1]]
+        w, b, pre_p, act_p = _pointers(net.w16), _pointers(net.b), _pointers(pre), _pointers(act)
+        _lib.check(_lib.load().hpx_net_forward(_lib.ptr(x), s, w, b, cout, pre_p, act_p, _lib.ptr(out),
+                                               _lib.stream_handle()))
+        return out, pre, act
+
     def step(self, first_drop: int, lr: float | None = None) -> torch.Tensor:
         """One Adam step on drops first_drop .. first_drop + drops_per_step; returns the loss, the mean
         over SNR points of the NMSE in dB (device scalar)."""
@@ -267,40 +285,32 @@ class Trainer:
         lib, st = _lib.load(), _lib.stream_handle()
         ls = self.simulate(first_drop)
         x = net.net_input(ls, self.noise_power)
-        out, cache = net.forward(x, keep=True)
-        grad = torch.empty_like(out)
+        out, pre, act = self._forward(x)
+        s, hidden = x.shape[0], len(net.shapes) - 1
+        dz = [torch.empty((s, POSITIONS, cout), dtype=torch.bfloat16, device=net.device) for _, cout, _ in net.shapes]
         group = torch.as_tensor(((first_drop + np.arange(self.drops)) % self.num_groups).astype(np.int32),
                                 device=net.device)
         self.work.zero_()
-        _lib.check(lib.hpx_nmse_grad(_lib.ptr(out), _lib.ptr(self.csi), _lib.ptr(self.spatial), self.drops, c.num_rx,
-                                     c.num_tx, c.words, c.num_subcarriers, _lib.ptr(group), self.num_groups,
-                                     _lib.ptr(self.work), _lib.ptr(grad), _lib.ptr(self.loss), st))
-        s = x.shape[0]
-        for i in range(len(net.shapes) - 1, -1, -1):
-            cin, cout, act = net.shapes[i]
-            a_in, pre = cache[i]
-            dz = torch.empty((s, POSITIONS, cout), dtype=torch.bfloat16, device=net.device)
-            if act:
-                _lib.check(lib.hpx_gelu_backward(_lib.ptr(grad), _lib.ptr(pre), grad.numel(), _lib.ptr(dz), st))
-            else:
-                _lib.check(lib.hpx_to_bf16(_lib.ptr(grad), grad.numel(), _lib.ptr(dz), st))
-            _lib.check(lib.hpx_conv1d_wgrad(_lib.ptr(dz), _lib.ptr(a_in), s, cin, cout, TAPS, DILATIONS[i],
-                                            _lib.ptr(self.workspace), _lib.ptr(self.gw[i]), _lib.ptr(self.gb[i]), st))
-            if i == len(net.shapes) - 1:  # the skip convolution sees the same output gradient
-                scin, scout = skip_shape(c)
-                _lib.check(lib.hpx_conv1d_wgrad(_lib.ptr(dz), _lib.ptr(x), s, scin, scout, SKIP_TAPS, 1,
-                                                _lib.ptr(self.workspace), _lib.ptr(self.gw[-1]), _lib.ptr(self.gb[-1]),
-                                                st))
-            if i > 0:
-                grad = torch.empty((s, POSITIONS, cin), dtype=torch.float32, device=net.device)
-                _lib.check(lib.hpx_conv1d_forward(_lib.ptr(dz), s, cout, TAPS, DILATIONS[i], _lib.ptr(net.wt16[i]), None,
-                                                  cin, 0, _lib.ptr(grad), None, st))
+        _lib.check(lib.hpx_nmse_grad_bf16(_lib.ptr(out), _lib.ptr(self.csi), _lib.ptr(self.spatial), self.drops, c.num_rx,
+                                          c.num_tx, c.words, c.num_subcarriers, _lib.ptr(group), self.num_groups,
+                                          _lib.ptr(self.work), _lib.ptr(dz[-1]), _lib.ptr(self.loss), st))
+        wt, pre_p, dz_p = _pointers(net.wt16[1:hidden + 1]), _pointers(pre), _pointers(dz[:hidden])
+        _lib.check(lib.hpx_net_backward(_lib.ptr(dz[-1]), s, net.shapes[-1][1], wt, pre_p, dz_p, st))
+        layers = [(dz[i], a_in, *net.shapes[i][:2], TAPS, DILATIONS[i]) for i, a_in in enumerate([x, *act])]
+        layers.append((dz[-1], x, *skip_shape(c), SKIP_TAPS, 1))  # the skip convolution sees the output's gradient
+        for i, (d, a_in, cin, cout, taps, dil) in enumerate(layers):
+            _lib.check(lib.hpx_conv1d_wgrad(_lib.ptr(d), _lib.ptr(a_in), s, cin, cout, taps, dil, _lib.ptr(self.workspace),
+                                            _lib.ptr(self.gw[i]), _lib.ptr(self.gb[i]), st))
         self.step_count += 1
         b1, b2 = self.betas
-        for p, g, m1, m2 in zip(net.w + net.b, self.gw + self.gb, self.m1, self.m2):
-            _lib.check(lib.hpx_adam_step(_lib.ptr(p), _lib.ptr(g), _lib.ptr(m1), _lib.ptr(m2), p.numel(),
-                                         float(self.lr if lr is None else lr), b1, b2, self.eps, self.step_count, st))
-        net.refresh()
+        copies = [(w16, wt16, w.shape[1], w.shape[2]) for w, w16, wt16 in zip(net.w, net.w16, net.wt16)]
+        tensors = (_lib.HpxAdamTensor * (len(net.w) + len(net.b)))(*[
+            _lib.HpxAdamTensor(_lib.ptr(p), _lib.ptr(g), _lib.ptr(m1), _lib.ptr(m2), _lib.ptr(w16), _lib.ptr(wt16),
+                               p.numel(), taps, cin)
+            for p, g, m1, m2, (w16, wt16, taps, cin) in zip(net.w + net.b, self.gw + self.gb, self.m1, self.m2,
+                                                            copies + [(None, None, 0, 0)] * len(net.b))])
+        _lib.check(lib.hpx_adam_steps(tensors, len(tensors), float(self.lr if lr is None else lr), b1, b2, self.eps,
+                                      self.step_count, st))
         return self.loss[0]
 
 

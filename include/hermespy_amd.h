@@ -430,6 +430,40 @@ int hpx_learned_estimate(const hpx_c64* grid, int64_t num_drops, int num_rx, int
                          const double* noise_power, const uint16_t* const* weights, const float* const* biases,
                          int cout, hpx_c64* est, void* stream);
 
+/* hpx_nmse_grad with the gradient rounded to bfloat16, as hpx_net_backward takes it. */
+int hpx_nmse_grad_bf16(const float* out, const hpx_c64* csi, const hpx_c64* spatial, int64_t num_drops, int num_rx,
+                       int num_tx, int words, int num_subcarriers, const int32_t* group, int num_groups, double* work,
+                       uint16_t* grad, double* loss, void* stream);
+
+/* Forward pass of a training step in one launch: x [num_samples][64][8] through the network of
+ * hpx_learned_estimate; pre[i] / act[i] (host arrays of 3 device pointers) [num_samples][64][64] are the
+ * hidden layers' pre-activations (float32) and activations (bfloat16), out [num_samples][64][cout]
+ * the output.  Arrays are 16-byte aligned. */
+int hpx_net_forward(const uint16_t* x, int64_t num_samples, const uint16_t* const* weights, const float* const* biases,
+                    int cout, float* const* pre, uint16_t* const* act, float* out, void* stream);
+
+/* Backward through the data in one launch: dz_out [num_samples][64][cout] (cout = 224) -> dz[i]
+ * [num_samples][64][64], the gradients of the hidden layers' pre-activations pre[i];
+ * weights_transposed: layers 2, 3, 4 as hpx_conv1d_weight_copies writes them.  Arrays are 16-byte aligned. */
+int hpx_net_backward(const uint16_t* dz_out, int64_t num_samples, int cout, const uint16_t* const* weights_transposed,
+                     const float* const* pre, uint16_t* const* dz, void* stream);
+
+/* hpx_adam_step of up to HPX_ADAM_MAX_TENSORS tensors in one launch; weight / weight_transposed (either may
+ * be NULL) receive the new parameters' bfloat16 copies of hpx_conv1d_weight_copies. */
+#define HPX_ADAM_MAX_TENSORS 16
+typedef struct hpx_adam_tensor {
+  float* param;
+  const float* grad;
+  float* m1;
+  float* m2;
+  uint16_t* weight;
+  uint16_t* weight_transposed; /* param is [cout][taps][cin] */
+  int64_t n;                   /* elements */
+  int32_t taps, cin;
+} hpx_adam_tensor;
+int hpx_adam_steps(const hpx_adam_tensor* tensors, int count, float lr, float beta1, float beta2, float eps,
+                   int64_t step, void* stream);
+
 /* One Adam step (bias-corrected, step >= 1) on float32 parameters. */
 int hpx_adam_step(float* param, const float* grad, float* m1, float* m2, int64_t n, float lr, float beta1, float beta2,
                   float eps, int64_t step, void* stream);

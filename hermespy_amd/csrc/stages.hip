@@ -104,14 +104,27 @@ constexpr int kMaxAntennas = 8;
 constexpr int kTdlThreads = 256;
 
 // One output sample per thread; Taylor coefficients of the block range the
-// workgroup touches live in LDS (direct evaluation when use_taylor == 0).
+// workgroup touches live in LDS (direct evaluation when use_taylor == 0).  STAGE: so does the window of x the
+// workgroup's paths reach, 256 + max_delay samples of every antenna, so that a path costs LDS reads and not a
+// trip to memory (4 antennas, 16 paths, one frame of 1024 subcarriers: 30 us, now 25: the rest is the coefficients).
+template <bool STAGE>
 __global__ void __launch_bounds__(kTdlThreads) tdl_propagate_kernel(
     const float2* __restrict__ x, int ntx, int64_t ld_x, int64_t m_len, const double* __restrict__ sos, int paths,
     int terms, int log2b, const int32_t* __restrict__ delays, int32_t max_delay, const float2* __restrict__ spatial,
     int nrx, float2* __restrict__ y, int64_t ld_y, int use_taylor) {
-  extern __shared__ float2 coeff[];  // [paths][nb][kTaylorCoeffs]
+  extern __shared__ float2 coeff[];  // [paths][nb][kTaylorCoeffs], STAGE: after the window [ntx][kTdlThreads + max_delay]
   const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kTdlThreads;
   const int64_t out_len = m_len + max_delay;
+  const int width = kTdlThreads + max_delay;
+  const float2* window = coeff;
+  float2* const coef = coeff + (STAGE ? ntx * width : 0);
+  if constexpr (STAGE) {
+    for (int t = 0; t < ntx; ++t)
+      for (int i = threadIdx.x; i < width; i += kTdlThreads) {
+        const int64_t m = n0 - max_delay + i;
+        coeff[t * width + i] = m >= 0 && m < m_len ? x[t * ld_x + m] : make_float2(0.f, 0.f);
+      }
+  }
   const TaylorBlocks tb{log2b};
   int64_t b_lo = 0;
   int nb = 0;
@@ -125,10 +138,10 @@ __global__ void __launch_bounds__(kTdlThreads) tdl_propagate_kernel(
     for (int i = threadIdx.x; i < paths * nb; i += kTdlThreads) {
       const int p = i / nb, b = i - p * nb;
       taylor_coeffs(sos + static_cast<int64_t>(p) * terms * 3, terms, tb.centre(b_lo + b), tb.half_width(),
-                    coeff + (p * nb + b) * kTaylorCoeffs);
+                    coef + (p * nb + b) * kTaylorCoeffs);
     }
-    __syncthreads();
   }
+  if (use_taylor || STAGE) __syncthreads();
   const int64_t n = n0 + threadIdx.x;
   if (n >= out_len) return;
   float2 z[kMaxAntennas];
@@ -141,13 +154,13 @@ __global__ void __launch_bounds__(kTdlThreads) tdl_propagate_kernel(
     float2 h;
     if (use_taylor) {
       const int b = static_cast<int>(tb.block_of(m) - b_lo);
-      h = taylor_eval(coeff + (p * nb + b) * kTaylorCoeffs, tb.offset(m));
+      h = taylor_eval(coef + (p * nb + b) * kTaylorCoeffs, tb.offset(m));
     } else {
       h = tap_direct(sos + static_cast<int64_t>(p) * terms * 3, terms, m);
     }
 #pragma unroll
     for (int t = 0; t < kMaxAntennas; ++t)
-      if (t < ntx) z[t] = cfma(h, x[t * ld_x + m], z[t]);
+      if (t < ntx) z[t] = cfma(h, STAGE ? window[t * width + max_delay + static_cast<int>(threadIdx.x) - d] : x[t * ld_x + m], z[t]);
   }
   for (int r = 0; r < nrx; ++r) {
     float2 acc = make_float2(0.f, 0.f);
@@ -183,7 +196,10 @@ extern "C" int hpx_tdl_propagate(const hpx_c64* x, int num_tx, int64_t ld_x, int
     }
   }
   const dim3 grid(static_cast<unsigned>((out_len + kTdlThreads - 1) / kTdlThreads));
-  hipLaunchKernelGGL(tdl_propagate_kernel, grid, dim3(kTdlThreads), lds, HPX_STREAM(stream),
+  const int64_t window = (static_cast<int64_t>(kTdlThreads) + max_delay) * num_tx * static_cast<int64_t>(sizeof(float2));
+  const bool stage = static_cast<int64_t>(lds) + window <= 64 * 1024;
+  if (stage) lds += static_cast<size_t>(window);
+  hipLaunchKernelGGL(stage ? tdl_propagate_kernel<true> : tdl_propagate_kernel<false>, grid, dim3(kTdlThreads), lds, HPX_STREAM(stream),
                      reinterpret_cast<const float2*>(x), num_tx, ld_x, num_samples, sos, num_paths, num_terms, log2b,
                      delays, max_delay, reinterpret_cast<const float2*>(spatial), num_rx, reinterpret_cast<float2*>(y),
                      ld_y, use_taylor);
@@ -495,25 +511,57 @@ extern "C" int hpx_ofdm_demodulate(const hpx_c64* frame, int num_streams, int64_
 // ------------------------------------------------------------------ ideal CSI
 constexpr int kCsiThreads = 256;
 
-// One workgroup per word: word means of every path (float64 Dirichlet form),
-// then one subcarrier per thread.
+// Workgroup (word, share of the subcarriers): word means of every path (float64 Dirichlet form), then one
+// subcarrier per thread.  The means' sines and cosines are the long part: with TERMS every (path, term)
+// pair has a thread and the path's sum runs over them in LDS in the same order; otherwise (tables beyond
+// kCsiTerms) a thread does its path's terms one after the other.  16 paths of 21 terms at 1024 subcarriers
+// and 14 words: 34 us with the terms in turn and a workgroup per word, 9.4 us now.
+constexpr int kCsiTerms = 1536;  // (path, term) pairs: 36 KB
+
+template <bool TERMS>
 __global__ void __launch_bounds__(kCsiThreads) ideal_csi_kernel(const double* __restrict__ sos, int paths, int terms,
                                                                 const int32_t* __restrict__ delays, int keep_below,
                                                                 const float2* __restrict__ spatial, int nrx, int ntx,
                                                                 int words, int n, int cp, int dc,
                                                                 float2* __restrict__ csi) {
-  extern __shared__ float2 lds[];
-  float2* abar = lds;           // [paths]
-  float2* tw = lds + paths;     // [n]
+  extern __shared__ double csi_lds[];
+  double* part = csi_lds;  // TERMS: [paths terms] weight, cosine, sine
+  float2* abar = reinterpret_cast<float2*>(csi_lds + (TERMS ? 3 * paths * terms : 0));  // [paths]
+  float2* tw = abar + paths;                                                         // [n]
   const int w = blockIdx.x;
   fill_twiddles(tw, n);
   const double m0 = static_cast<double>(w) * (n + cp) + cp;
-  for (int p = threadIdx.x; p < paths; p += kCsiThreads) {
-    const double2 a = tap_mean(sos + static_cast<int64_t>(p) * terms * 3, terms, m0, n);
-    abar[p] = make_float2(static_cast<float>(a.x), static_cast<float>(a.y));
+  if constexpr (TERMS) {
+    const double centre = m0 + 0.5 * static_cast<double>(n - 1);
+    for (int e = threadIdx.x; e < paths * terms; e += kCsiThreads) {
+      const double rate = sos[3 * e], amp = sos[3 * e + 2];
+      double s = 0.0, c = 0.0, weight = 0.0;
+      if (amp != 0.0) {
+        weight = amp * dirichlet_factor(rate, n);
+        sincos(reduce_phase(fma(rate, centre, sos[3 * e + 1])), &s, &c);
+      }
+      part[3 * e] = weight;
+      part[3 * e + 1] = c;
+      part[3 * e + 2] = s;
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < paths; p += kCsiThreads) {
+      double ar = 0.0, ai = 0.0;
+      for (int k = 0; k < terms; ++k) {
+        const double* t = part + 3 * (p * terms + k);
+        ar = fma(t[0], t[1], ar);
+        ai = fma(t[0], t[2], ai);
+      }
+      abar[p] = make_float2(static_cast<float>(ar), static_cast<float>(ai));
+    }
+  } else {
+    for (int p = threadIdx.x; p < paths; p += kCsiThreads) {
+      const double2 a = tap_mean(sos + static_cast<int64_t>(p) * terms * 3, terms, m0, n);
+      abar[p] = make_float2(static_cast<float>(a.x), static_cast<float>(a.y));
+    }
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < n; q += kCsiThreads) {
+  for (int q = static_cast<int>(blockIdx.y) * kCsiThreads + threadIdx.x; q < n; q += static_cast<int>(gridDim.y) * kCsiThreads) {
     const int bin = subcarrier_bin(q, n, dc);
     float2 c = make_float2(0.f, 0.f);
     for (int p = 0; p < paths; ++p) {
@@ -541,10 +589,15 @@ extern "C" int hpx_ideal_csi(const double* sos, int num_paths, int num_terms, co
                   prefix >= 0 && num_taps >= 1,
               "hpx_ideal_csi: invalid sizes");
   const int keep_below = std::min<int>(num_taps, num_subcarriers);
-  const size_t lds = (static_cast<size_t>(num_paths) + num_subcarriers) * sizeof(float2);
-  hipLaunchKernelGGL(ideal_csi_kernel, dim3(words), dim3(kCsiThreads), lds, HPX_STREAM(stream), sos, num_paths,
-                     num_terms, delays, keep_below, reinterpret_cast<const float2*>(spatial), num_rx, num_tx, words,
-                     num_subcarriers, prefix, dc_suppression, reinterpret_cast<float2*>(csi));
+  size_t lds = (static_cast<size_t>(num_paths) + num_subcarriers) * sizeof(float2);
+  const bool by_term = static_cast<int64_t>(num_paths) * num_terms <= kCsiTerms &&
+                       lds + 3 * sizeof(double) * num_paths * num_terms <= 64 * 1024;
+  if (by_term) lds += 3 * sizeof(double) * num_paths * num_terms;
+  const dim3 g(static_cast<unsigned>(words), static_cast<unsigned>((num_subcarriers + kCsiThreads - 1) / kCsiThreads));
+  hipLaunchKernelGGL(by_term ? ideal_csi_kernel<true> : ideal_csi_kernel<false>, g, dim3(kCsiThreads), lds,
+                     HPX_STREAM(stream), sos, num_paths, num_terms, delays, keep_below,
+                     reinterpret_cast<const float2*>(spatial), num_rx, num_tx, words, num_subcarriers, prefix,
+                     dc_suppression, reinterpret_cast<float2*>(csi));
   return check_launch("hpx_ideal_csi");
 }
 
@@ -612,24 +665,39 @@ extern "C" int hpx_equalize(const hpx_c64* y, const hpx_c64* h, int num_rx, int 
 }
 
 // ------------------------------------------------------------------ bit errors
+// 16 bytes per thread and step where both arrays allow it, one atomic per workgroup: all of them go to one
+// address, which bounded the kernel (a wavefront's 256 bytes an atomic: 344064 bits 12.4 us, 2.9 now).
 __global__ void __launch_bounds__(256) count_errors_kernel(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                                                            int64_t n, unsigned long long* __restrict__ errors) {
+  __shared__ unsigned long long red[4];
   unsigned long long local = 0;
-  const int64_t words = n / 4;
-  const uint32_t* aw = reinterpret_cast<const uint32_t*>(a);
-  const uint32_t* bw = reinterpret_cast<const uint32_t*>(b);
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const bool aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 3u) == 0;
-  if (aligned) {
-    for (int64_t i = tid; i < words; i += stride) local += __popc((aw[i] ^ bw[i]) & 0x01010101u);
-    for (int64_t i = words * 4 + tid; i < n; i += stride) local += ((a[i] ^ b[i]) & 1u);
-  } else {
-    for (int64_t i = tid; i < n; i += stride) local += ((a[i] ^ b[i]) & 1u);
+  const uintptr_t both = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b);
+  int64_t rest = 0;  // bits from here are compared one by one
+  if ((both & 15u) == 0) {
+    const uint4* aw = reinterpret_cast<const uint4*>(a);
+    const uint4* bw = reinterpret_cast<const uint4*>(b);
+    for (int64_t i = tid; i < n / 16; i += stride) {
+      const uint4 x = aw[i], y = bw[i];
+      local += __popc((x.x ^ y.x) & 0x01010101u) + __popc((x.y ^ y.y) & 0x01010101u) +
+               __popc((x.z ^ y.z) & 0x01010101u) + __popc((x.w ^ y.w) & 0x01010101u);
+    }
+    rest = n / 16 * 16;
+  } else if ((both & 3u) == 0) {
+    const uint32_t* aw = reinterpret_cast<const uint32_t*>(a);
+    const uint32_t* bw = reinterpret_cast<const uint32_t*>(b);
+    for (int64_t i = tid; i < n / 4; i += stride) local += __popc((aw[i] ^ bw[i]) & 0x01010101u);
+    rest = n / 4 * 4;
   }
-  // wavefront reduction then one atomic per wave
+  for (int64_t i = rest + tid; i < n; i += stride) local += ((a[i] ^ b[i]) & 1u);
   for (int off = 32; off > 0; off >>= 1) local += __shfl_down(local, off, 64);
-  if ((threadIdx.x & 63) == 0 && local) atomicAdd(errors, local);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = local;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    local = (red[0] + red[1]) + (red[2] + red[3]);
+    if (local) atomicAdd(errors, local);
+  }
 }
 
 extern "C" int hpx_count_errors(const uint8_t* a, const uint8_t* b, int64_t num_bits, unsigned long long* errors,
@@ -637,7 +705,8 @@ extern "C" int hpx_count_errors(const uint8_t* a, const uint8_t* b, int64_t num_
   HPX_REQUIRE(num_bits >= 0, "hpx_count_errors: negative length");
   if (num_bits == 0) return HPX_OK;
   HPX_REQUIRE(a && b && errors, "hpx_count_errors: null pointer");
-  const int64_t work = std::max<int64_t>(1, num_bits / 4);
+  const bool vec = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15u) == 0;
+  const int64_t work = std::max<int64_t>(1, num_bits / (vec ? 16 : 4));
   const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((work + 255) / 256, 4096));
   hipLaunchKernelGGL(count_errors_kernel, dim3(blocks), dim3(256), 0, HPX_STREAM(stream), a, b, num_bits, errors);
   return check_launch("hpx_count_errors");
@@ -656,15 +725,21 @@ extern "C" int hpx_spatial_detector_host(int num_rx, int num_tx, const hpx_c128*
 }
 
 // ------------------------------------------------------------------ random streams
+// 16 bits per thread, stored as one 16-byte piece (eight threads draw the same Philox call; one thread per call
+// storing its 128 bytes one by one took 18 us for any frame, latency alone: 2.6 us now for 86016 bits).
 __global__ void __launch_bounds__(256) stream_bits_kernel(uint64_t seed, uint32_t drop, uint32_t stream_id,
                                                           int64_t nbits, uint8_t* __restrict__ bits) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;  // one Philox call = 128 bits
-  if (c * 128 >= nbits) return;
-  const uint4 w = stream_call(seed, drop, stream_id, static_cast<uint32_t>(c));
-  const uint32_t comp[4] = {w.x, w.y, w.z, w.w};
-  for (int k = 0; k < 128; ++k) {
-    const int64_t i = c * 128 + k;
-    if (i < nbits) bits[i] = static_cast<uint8_t>((comp[k >> 5] >> (k & 31)) & 1u);
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 16;
+  if (i >= nbits) return;
+  const uint4 w = stream_call(seed, drop, stream_id, static_cast<uint32_t>(i >> 7));
+  const int k = static_cast<int>(i >> 5) & 3;
+  const uint32_t v = (k == 0 ? w.x : k == 1 ? w.y : k == 2 ? w.z : w.w) >> (i & 16);
+  // four bits to the lowest bits of four bytes
+  auto spread = [](uint32_t four) { return ((four & 15u) * 0x00204081u) & 0x01010101u; };
+  if (i + 16 <= nbits && (reinterpret_cast<uintptr_t>(bits) & 15u) == 0) {
+    *reinterpret_cast<uint4*>(bits + i) = make_uint4(spread(v), spread(v >> 4), spread(v >> 8), spread(v >> 12));
+  } else {
+    for (int j = 0; j < 16 && i + j < nbits; ++j) bits[i + j] = static_cast<uint8_t>((v >> j) & 1u);
   }
 }
 
@@ -673,8 +748,8 @@ extern "C" int hpx_stream_bits(uint64_t seed, uint32_t drop, uint32_t stream_id,
   HPX_REQUIRE(num_bits >= 0 && num_bits <= (int64_t(1) << 38), "hpx_stream_bits: invalid length");
   if (num_bits == 0) return HPX_OK;
   HPX_REQUIRE(bits, "hpx_stream_bits: null pointer");
-  const int64_t calls = (num_bits + 127) / 128;
-  hipLaunchKernelGGL(stream_bits_kernel, dim3(static_cast<unsigned>((calls + 255) / 256)), dim3(256), 0,
+  const int64_t pieces = (num_bits + 15) / 16;
+  hipLaunchKernelGGL(stream_bits_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
                      HPX_STREAM(stream), seed, drop, stream_id, num_bits, bits);
   return check_launch("hpx_stream_bits");
 }

@@ -141,6 +141,8 @@ __device__ __forceinline__ uint32_t symbol_bits(const uint32_t* bw, int bit, int
 // local_drop indexes the per-drop arrays (noise power, Doppler, errors, exports); the Philox drop
 // index is drop_index[local_drop] or first_drop + local_drop.  Segments of a drop add their bit errors
 // to errors[local_drop], which is zero before; a drop alone (segs = 1) stores its count.
+// LEAN: the segments of a drop (segs > 1) share its device workspace and only read it; a launch with
+// segs = 0 before them fills it (Taylor table, twiddles, FFT pass table) and zeroes the drop's errors.
 // BATCH: a.wb words go through every step at once (rows [word][stream], then the words' CSI rows), so
 // that a drop of few subcarriers fills its wavefronts and takes a barrier per step and batch instead
 // of per step and word.  Every value is computed by the same expression whatever the batch, the
@@ -183,8 +185,11 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
   const int L = a.paths;
   const int period = n + a.cp;
   // this workgroup's words, and the Taylor blocks their windows and delays reach
-  const int w_begin = static_cast<int>(static_cast<int64_t>(a.words) * seg / segs);
-  const int w_end = static_cast<int>(static_cast<int64_t>(a.words) * (seg + 1) / segs);
+  const bool tables_only = LEAN && segs == 0;
+  const bool fill_tables = !LEAN || segs <= 1;
+  const int parts = LEAN && segs == 0 ? 1 : segs;
+  const int w_begin = static_cast<int>(static_cast<int64_t>(a.words) * seg / parts);
+  const int w_end = static_cast<int>(static_cast<int64_t>(a.words) * (seg + 1) / parts);
   const int b_first = max(0, w_begin * period + a.cp - a.maxd) >> a.log2b;
   const int b_count = ((w_end * period - 1) >> a.log2b) + 1 - b_first;
   // Taylor table [path][a.nb blocks from b_first], indexed by the block itself
@@ -329,7 +334,7 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
     const double2 p = constellation_point(a.order, 1, bits_to_label(static_cast<uint32_t>(v), a.bps));
     cons[v] = make_float2(static_cast<float>(p.x * a.tx_scale), static_cast<float>(p.y * a.tx_scale));
   }
-  fill_fft_pass_table(ptab, a.log2n);
+  if (fill_tables) fill_fft_pass_table(ptab, a.log2n);
   if (tid == 0) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -337,7 +342,7 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
       dmb->b[i] = a.dbounds.b[i];
     }
   }
-  if (LEAN) {
+  if (LEAN && fill_tables) {
     for (int k = tid; k < n; k += nthreads) {
       double s, c;
       sincospi(-2.0 * static_cast<double>(k) / static_cast<double>(n), &s, &c);
@@ -353,7 +358,7 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
   // wavefront does both in turn).
   const bool split = nthreads >= 128;
   const int det_first = split ? nthreads - 64 : 0;
-  if (tid >= det_first) {
+  if (tid >= det_first && !tables_only) {
     double* lam = s64 + 2 * NR * NT;
     double* v = lam + NT;
     double* am = v + 2 * NT * NT;
@@ -370,7 +375,7 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
     for (int i = lane; i < NT; i += 64) det_l[i] = lam[i] > rt * rt * lmax ? static_cast<float>(lam[i]) : 0.0f;
   }
   const int taylor_threads = split ? det_first : nthreads;
-  if (tid < taylor_threads) {
+  if (tid < taylor_threads && fill_tables) {
     for (int e = tid; e < L * b_count; e += taylor_threads) {
       const int p = e / b_count, b = b_first + (e - p * b_count);
       float2* c = coef0 + (p * a.nb + b) * kTaylorCoeffs;
@@ -381,6 +386,10 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
         for (int k = 0; k < kTaylorCoeffs; ++k) c[k] = make_float2(0.f, 0.f);
       }
     }
+  }
+  if (tables_only) {
+    if (tid == 0) global(a.errors)[local_drop] = 0;
+    return;
   }
   for (int e = tid; e < L * (w_end - w_begin); e += nthreads) {
     const int p = e / (w_end - w_begin), w = w_begin + (e - p * (w_end - w_begin));
@@ -728,8 +737,9 @@ batch_kernel(BatchArgs a, int segs) {
 template <int NT, int NR, int PAIRS, int MAXT, bool LEAN = false, int FFTV = fft_values<NT, MAXT>(), bool BATCH = false>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(batch_waves_per_eu<NT, PAIRS, MAXT>())))
 batch_kernel_multi(const BatchArgs* __restrict__ plans, int segs) {
-  const int slot = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / segs);
-  drop_body<NT, NR, PAIRS, FFTV, LEAN, true, BATCH>((ConstArgs*)(plans + slot), 0, static_cast<int>(blockIdx.x) - slot * segs, segs);
+  const int parts = LEAN && segs == 0 ? 1 : segs;
+  const int slot = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / parts);
+  drop_body<NT, NR, PAIRS, FFTV, LEAN, true, BATCH>((ConstArgs*)(plans + slot), 0, static_cast<int>(blockIdx.x) - slot * parts, segs);
 }
 
 // Zero error counts of drops whose segments add to them (a kernel, so that a captured graph holds no
@@ -793,7 +803,11 @@ int segments_for(int64_t drops, int most, Resident resident) {
   }
   return best;
 }
-constexpr int kMultiMaxSegments = 7;  // (a class's words per drop are known to its plans only)
+// (A class's words per drop are known to its plans only.)  Lean drops, one of which a CU holds and which take
+// 1.5 ms each in one piece, are cut too, after a launch that fills their workspaces: mixed batches of 64, 300,
+// 1000 and 2048 drops 1763, 3207, 2373 and 3076 us with lean drops whole, 844, 1272, 1620 and 2904 us in up to
+// four segments, 652, 897, 1631 and 2963 us in up to seven.
+constexpr int kMultiMaxSegments = 7;
 
 // Raises a kernel's dynamic LDS limit once per process and size (so that launches recorded
 // into a graph after a first eager run make no attribute calls).
@@ -828,11 +842,12 @@ int launch_multi_kernel(const BatchArgs* plans, const hpx_uneven_class& c, hipSt
   }
   const BatchArgs* first = plans + c.first;
   const int threads = batched_class(NT, c.threads, c.pairs) ? batch_threads(NT) : c.threads;
-  // (the segments of a lean drop would share its workspace)
   const int64_t resident =
       resident_workgroups(waves_per_cu(reinterpret_cast<const void*>(fn)), threads, c.lds_bytes);
-  const int segs = LEAN ? 1 : segments_for(c.count, kMultiMaxSegments, [&](int) { return resident; });
-  if (segs > 1)
+  const int segs = segments_for(c.count, kMultiMaxSegments, [&](int) { return resident; });
+  if (LEAN && segs > 1)  // the workspaces first
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(c.count)), dim3(threads), c.lds_bytes, stream, first, 0);
+  else if (segs > 1)
     hipLaunchKernelGGL(zero_plan_errors_kernel, dim3(static_cast<unsigned>((c.count + 255) / 256)), dim3(256), 0, stream,
                        first, static_cast<int>(c.count));
   hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(c.count * segs)), dim3(threads), c.lds_bytes, stream, first, segs);

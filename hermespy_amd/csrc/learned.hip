@@ -455,7 +455,7 @@ __device__ __forceinline__ int64_t out_index(int64_t s, int e, int words, int n)
 // Threads 256 apart differ by a fixed (position, word, subcarrier) step, so the pair's place is carried along
 // instead of divided out each time, and reads of the output and writes of the gradient are whole lines:
 // 4096 samples of 224 channels 90 us, bfloat16 gradients (159 us, and 117 us for the conversion, before).
-// (The accumulation keeps the grid's order, in which the channel is read in whole lines: 89 us, 129 in this one.)
+// (The accumulation keeps the grid's order and so the order of its sums: 128 us, 129 in this one.)
 struct PairWalk {
   int p, w, u;  // position, word, subcarrier of the position: subcarrier blk p + u of word w
   int dp, dw, du, blk, words;
@@ -867,11 +867,23 @@ net_forward_kernel(const float2* __restrict__ grid, int num_drops, int num_rx, i
         if (s0 + g < num_samples) {
           const int64_t o = ((s0 + g) * kPos + p) * 64 + co;
           *reinterpret_cast<floatx4*>(kept.pre[layer] + o) = v;
-          *reinterpret_cast<bf16x4n*>(kept.act[layer] + o) = h;
         }
       }
     });
     sample_sync<PT>();
+    // the activations from LDS, in whole lines (eight bytes a lane from the accumulators touch 32 lines a store: a
+    // training forward pass of 4096 samples 332 us, 287 now)
+    if constexpr (TRAIN) {
+      constexpr int kLanes = PT == 1 ? 128 : 64;
+      const int g = ln.template sample<PT>(0);
+      if (s0 + g < num_samples) {
+        uint16_t* dst = kept.act[layer] + (s0 + g) * kActElems;
+#pragma unroll
+        for (int i = tid & (kLanes - 1); i < kActElems / 8; i += kLanes)
+          *reinterpret_cast<uintx4*>(dst + 8 * i) =
+              *reinterpret_cast<const uintx4*>(act + g * kActElems + act_at(i >> 3, 8 * (i & 7)));
+      }
+    }
   };
   {
     floatx16 acc[2][PT];

@@ -182,165 +182,183 @@ __global__ void __launch_bounds__(256) wgrad_kernel(const uint16_t* __restrict__
   }
 }
 
-// The same partial sums on the matrix cores: the gradient is the product of dz^T (cout x positions)
-// with the im2col rows of the input (positions x (tap, ci)), contracted over the positions of the
-// chunk's samples in 32x32x16 bf16 MFMAs with float32 accumulation.  Both operands need eight
-// consecutive positions per lane while memory holds channels innermost, so the fragments come
-// through the transposing LDS read (each lane names the row it wants read, so a tap's circular
-// shift is only another row index and no im2col copy exists).  One more column of ones makes the
-// bias gradient.  A workgroup holds one sample's dz and input rows in LDS (the next sample's are in
-// flight in registers) and each of its four wavefronts a strip of COT x 32 output channels by 32
-// columns in accumulators: 2 COT + 2 fragment reads feed COT MFMAs.  Row strides of 32 bytes mod
-// 128 spread the four rows a transposing read touches over all banks.  Bound: LDS fill from L2 (36 KB
-// a sample and workgroup at 64 -> 224 channels).  4096 samples on MI355X: 64 -> 224 channels
-// 68 us, 8 -> 224 with 17 taps 43 us, 64 -> 64 30 us (the VALU kernel above: 1546, 931 and 457 us).
-constexpr int kWgWaves = 4;
-
-template <int COT>
-constexpr int wgrad_dz_stride() {  // elements; bytes = 32 mod 128
-  return COT * 32 + (COT % 2 == 0 ? 16 : 48);
-}
-__host__ __device__ constexpr int wgrad_x_stride(int cin) { return cin >= 32 ? cin + 16 : cin; }
+// The same partial sums, bit for bit, on the float32 matrix cores.  A K = 1 MFMA adds one product to every
+// accumulator with one rounding, so a chain of them over the chunk's positions is the chain of fmas above (a
+// bf16 MFMA, three times as fast here, sums 16 products in an order of its own; Adam carries that into the
+// weights, activations round to other bfloat16 values, and the losses that follow leave the tenth digit).
+// v_mfma_f32_16x16x1_4b makes four 16 x 16 blocks at once: a wavefront owns four blocks (16 output channels by 16
+// (tap, ci) columns), the blocks of a workgroup's co group numbered channels first, so any four share an
+// instruction and no shape pads more than its last one.  A workgroup holds one
+// sample's dz columns and input rows in LDS (the next sample's are in flight in registers); memory holds
+// channels innermost, so the operands come through the transposing LDS read, four positions of a lane's channel at a time
+// (one read per position and operand took twice as long).  The input rows lie there twice, so that a tap's
+// circular shift is a fixed distance from the position and all 64 steps read at constant offsets.  Each row ends
+// in ones, the column of the bias gradient.
+// Bound: float32 MFMA, 32 cycles a step and wavefront, and whole rounds of the 1024 SIMDs.  4096 samples on
+// MI355X: 64 -> 224 channels 430 us, 8 -> 224 with 17 taps 177 us, 64 -> 64 133 us (the VALU kernel above: 1546, 931 and 457 us).
+// Wavefronts of a workgroup: eight where its dz columns take most of the LDS, so that a CU holds 16 (64 -> 224, 4096
+// samples: 430 us, with four 503), else four, which spread evenly over the CUs (64 -> 64: 133 us, with eight 164).
+constexpr int wgrad_waves(int cot) { return cot > 2 ? 8 : 4; }
 
 typedef short shortx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
 
-// elements 4 h .. 4 h + 3 along the rows for this lane's column; `p`: this lane's row and 4 columns
-__device__ __forceinline__ shortx4 lds_read_tr(const uint16_t* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)p);
+// Row strides in elements: 32 bytes mod 128, so that the four rows of a transposing read lie on different banks.
+constexpr int wgrad_dz_stride(int cot) { return cot * 32 + (cot % 2 == 0 ? 16 : 48); }
+constexpr int kWgXStride = 64 + 16;  // (the ones behind the channels)
+
+// Four rows of this lane's column of a 16-column tile per 16 lanes; `p`: the row (lane / 4) % 4 and the columns
+// from 4 (lane % 4) of the tile that this lane names.
+__device__ __forceinline__ uintx2 lds_read_tr(const uint16_t* p) {
+  return __builtin_bit_cast(uintx2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_shortx4*)p));
 }
 
+// COT: 32-channel tiles of a workgroup's co group.
 template <int COT>
-__global__ void __launch_bounds__(64 * kWgWaves) __attribute__((amdgpu_waves_per_eu(2)))
-wgrad_mfma_kernel(const uint16_t* __restrict__ dz,
+__global__ void __launch_bounds__(64 * wgrad_waves(COT)) wgrad_mfma_kernel(const uint16_t* __restrict__ dz,
                                                                   const uint16_t* __restrict__ in, int num_samples,
                                                                   int cout, int cin, int taps, int dil,
                                                                   float* __restrict__ part,
                                                                   float* __restrict__ part_bias) {
-  constexpr int DS = wgrad_dz_stride<COT>();
-  constexpr int kThreads = 64 * kWgWaves;
-  constexpr int kDzVecs = kPos * COT * 32 / 8 / kThreads;  // 16-byte vectors per thread: COT
-  constexpr int kXVecs = kPos * 64 / 8 / kThreads;         // at most 64 input channels
+  constexpr int DS = wgrad_dz_stride(COT);
+  constexpr int kWaves = wgrad_waves(COT), kThreads = 64 * kWaves;
+  constexpr int kDzVecs = kPos * COT * 32 / 8;  // 16-byte vectors of a sample's dz
+  constexpr int kDzEach = (kDzVecs + kThreads - 1) / kThreads;
+  constexpr int kXEach = kPos * 64 / 8 / kThreads;  // at most 64 input channels
   extern __shared__ __align__(16) uint16_t wg_lds[];
   uint16_t* dzs = wg_lds;
   uint16_t* xs = dzs + kPos * DS;
-  const int xstride = wgrad_x_stride(cin);
-  uint16_t* ones = xs + kPos * xstride;
+  constexpr int XS = kWgXStride;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int co0 = blockIdx.y * COT * 32;
   const int kcols = taps * cin;
-  const int kc0 = (blockIdx.z * kWgWaves + wave) * 32;
   const int chunk = blockIdx.x;
-  const int s_end = std::min(num_samples, (chunk + 1) * kWgSamples);
-  if (tid < 4) ones[tid] = 0x3f80;  // bf16 1
-  // the rows and columns this lane names in a transposing read: rows (lane / 4) % 4 of a group of
-  // four, four columns from 4 (lane % 4) of a group of 16; lanes 16.. take the next 16 columns,
-  // lanes 32.. the next eight rows
-  const int row4 = (lane >> 2) & 3, kq = lane >> 5;
-  const int cols = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  const int col = kc0 + cols;
-  const int tap = col / cin, ci = col - tap * cin;
-  const bool real = tap < taps;  // otherwise the bias column (and padding)
-  const int shift = (tap - taps / 2) * dil;
-  const uint16_t* xcol = real ? xs + ci : ones;
-  const int xmul = real ? xstride : 0;
-  const uint16_t* dzrow = dzs + (8 * kq + row4) * DS + cols;
+  const int s_begin = chunk * kWgSamples;
+  const int s_end = std::min(num_samples, s_begin + kWgSamples);
+  // the rows and columns this lane names in the transposing reads of its block (channel and (tap, ci) tile); the
+  // columns from kcols are ones: the bias column, and padding, which is dropped
+  constexpr int kCoBlocks = 2 * COT;
+  const int col_blocks = kcols / 16 + 1;
+  const int first_block = 4 * (static_cast<int>(blockIdx.z) * kWaves + wave);
+  const bool active = first_block < kCoBlocks * col_blocks;  // (whole wavefronts)
+  const int block = std::min(first_block + (lane >> 4), kCoBlocks * col_blocks - 1);
+  const int row4 = (lane >> 2) & 3;
+  const int col = 16 * (block / kCoBlocks) + 4 * (lane & 3);
+  const bool real = col < kcols;
+  const int tap = real ? col / cin : 0;
+  const uint16_t* az = dzs + row4 * DS + 16 * (block % kCoBlocks) + 4 * (lane & 3);
+  const uint16_t* bx =
+      xs + (row4 + (real ? ((tap - taps / 2) * dil) & (kPos - 1) : 0)) * XS + (real ? col - tap * cin : cin);
+  for (int i = tid; i < 2 * kPos * 4; i += kThreads) xs[(i >> 2) * XS + cin + (i & 3)] = 0x3f80;  // bf16 1
 
-  uintx4 rdz[kDzVecs], rx[kXVecs];
+  uintx4 rdz[kDzEach], rx[kXEach];
   const int xvecs = kPos * cin / 8;
   auto load = [&](int s) __attribute__((always_inline)) {
     const uint16_t* d = dz + static_cast<int64_t>(s) * kPos * cout + co0;
 #pragma unroll
-    for (int i = 0; i < kDzVecs; ++i) {
-      const int v = tid + i * kThreads;
+    for (int i = 0; i < kDzEach; ++i) {
+      const int v = std::min(tid + i * kThreads, kDzVecs - 1);
       const int p = v / (COT * 4), c = v - p * (COT * 4);
       rdz[i] = *reinterpret_cast<const uintx4*>(d + p * cout + 8 * c);
     }
     const uintx4* x = reinterpret_cast<const uintx4*>(in + static_cast<int64_t>(s) * kPos * cin);
 #pragma unroll
-    for (int i = 0; i < kXVecs; ++i) rx[i] = x[std::min(tid + i * kThreads, xvecs - 1)];
+    for (int i = 0; i < kXEach; ++i) rx[i] = x[std::min(tid + i * kThreads, xvecs - 1)];
   };
-  floatx16 acc[COT];
+  floatx16 acc;
 #pragma unroll
-  for (int t = 0; t < COT; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
   const int xrow_vecs = cin / 8;
-  load(chunk * kWgSamples);
-  for (int s = chunk * kWgSamples; s < s_end; ++s) {
+  load(s_begin);
+  for (int s = s_begin; s < s_end; ++s) {
 #pragma unroll
-    for (int i = 0; i < kDzVecs; ++i) {
+    for (int i = 0; i < kDzEach; ++i) {
       const int v = tid + i * kThreads;
       const int p = v / (COT * 4), c = v - p * (COT * 4);
-      *reinterpret_cast<uintx4*>(dzs + p * DS + 8 * c) = rdz[i];
+      if (v < kDzVecs) *reinterpret_cast<uintx4*>(dzs + p * DS + 8 * c) = rdz[i];
     }
 #pragma unroll
-    for (int i = 0; i < kXVecs; ++i) {
+    for (int i = 0; i < kXEach; ++i) {
       const int v = tid + i * kThreads;
       if (v < xvecs) {
         const int p = v / xrow_vecs, c = v - p * xrow_vecs;
-        *reinterpret_cast<uintx4*>(xs + p * xstride + 8 * c) = rx[i];
+        *reinterpret_cast<uintx4*>(xs + p * XS + 8 * c) = rx[i];
+        *reinterpret_cast<uintx4*>(xs + (p + kPos) * XS + 8 * c) = rx[i];
       }
     }
     __syncthreads();
     if (s + 1 < s_end) load(s + 1);
-    if (kc0 <= kcols) {
+    if (active) {
+      // 16 positions' operands are read while those before them are multiplied
+      constexpr int kReads = 4, kBatches = kPos / (4 * kReads);
+      uintx2 a[2][kReads], b[2][kReads];
+      auto read = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
-      for (int ks = 0; ks < kPos / 16; ++ks) {
-        shortx4 b[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int p = (16 * ks + 8 * kq + 4 * h + row4 + shift) & (kPos - 1);
-          b[h] = lds_read_tr(xcol + p * xmul);
+        for (int j = 0; j < kReads; ++j) {
+          a[q & 1][j] = lds_read_tr(az + 4 * (kReads * q + j) * DS);
+          b[q & 1][j] = lds_read_tr(bx + 4 * (kReads * q + j) * XS);
         }
-        const bf16x8 bv = __builtin_bit_cast(bf16x8, __builtin_shufflevector(b[0], b[1], 0, 1, 2, 3, 4, 5, 6, 7));
+      };
+      auto value = [](uintx2 v, int i) __attribute__((always_inline)) {
+        return __uint_as_float(i & 1 ? v[i >> 1] & 0xffff0000u : v[i >> 1] << 16);
+      };
+      read(0);
 #pragma unroll
-        for (int t = 0; t < COT; ++t) {
-          const shortx4 a0 = lds_read_tr(dzrow + 16 * ks * DS + 32 * t);
-          const shortx4 a1 = lds_read_tr(dzrow + (16 * ks + 4) * DS + 32 * t);
-          const bf16x8 av = __builtin_bit_cast(bf16x8, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[t], 0, 0, 0);
-        }
+      for (int q = 0; q < kBatches; ++q) {
+        if (q + 1 < kBatches) read(q + 1);
+        __builtin_amdgcn_sched_barrier(0);  // (the compiler would read each operand where it is used)
+#pragma unroll
+        for (int j = 0; j < kReads; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(value(a[q & 1][j], i), value(b[q & 1][j], i), acc, 0, 0, 0);
       }
     }
     __syncthreads();
   }
-  const int oc = kc0 + (lane & 31);
-  if (oc > kcols) return;
+  if (!active) return;
 #pragma unroll
-  for (int t = 0; t < COT; ++t)
+  for (int b = 0; b < 4; ++b) {
+    const int bl = first_block + b;
+    if (bl >= kCoBlocks * col_blocks) break;
+    const int oc = 16 * (bl / kCoBlocks) + (lane & 15);
+    if (oc > kcols) continue;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int co = co0 + 32 * t + 8 * (r >> 2) + 4 * kq + (r & 3);
-      const int64_t row = static_cast<int64_t>(chunk) * cout + co;
-      if (oc < kcols) part[row * kcols + oc] = acc[t][r];
-      else part_bias[row] = acc[t][r];
+    for (int r = 0; r < 4; ++r) {
+      const int64_t row = static_cast<int64_t>(chunk) * cout + co0 + 16 * (bl % kCoBlocks) + 4 * (lane >> 4) + r;
+      if (oc < kcols) part[row * kcols + oc] = acc[4 * b + r];
+      else part_bias[row] = acc[4 * b + r];
     }
+  }
 }
 
-// out[i] = sum of the chunks' partials of entry i, weights then biases: 64 entries per workgroup, its four
-// wavefronts each summing every fourth chunk (one thread per entry and all chunks in one chain was
-// latency-bound: 31 us for 128 chunks of any size, 5 to 7 us now).
+// out[i] = sum of the chunks' partials of entry i in their order, weights then biases.  One thread per entry; 32
+// chunks' values are read ahead of their additions, which are one chain (read one by one they were
+// latency-bound: 31 us for 128 chunks of any size, 5 us now).
 __global__ void __launch_bounds__(256) reduce_parts_kernel(const float* __restrict__ part_w, int64_t nw,
                                                            const float* __restrict__ part_b, int64_t nb, int chunks,
                                                            float* __restrict__ grad_w, float* __restrict__ grad_b) {
-  __shared__ float red[3][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + lane;
+  int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= nw + nb) return;
   const bool weight = i < nw;
   const int64_t n = weight ? nw : nb;
-  const float* part = weight ? part_w : part_b;
-  float* out = weight ? grad_w : grad_b;
   if (!weight) i -= nw;
+  const float* part = (weight ? part_w : part_b) + i;
+  constexpr int kAhead = 32;
   float s = 0.0f;
-  if (i < n) {
-#pragma unroll 8
-    for (int c = wave; c < chunks; c += 4) s += part[static_cast<int64_t>(c) * n + i];
+  int c = 0;
+  for (; c + kAhead <= chunks; c += kAhead) {
+    float v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) v[j] = part[static_cast<int64_t>(c + j) * n];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) s += v[j];
   }
-  if (wave) red[wave - 1][lane] = s;
-  __syncthreads();
-  if (wave == 0 && i < n) out[i] = (s + red[0][lane]) + (red[1][lane] + red[2][lane]);
+#pragma unroll 4
+  for (; c < chunks; ++c) s += part[static_cast<int64_t>(c) * n];
+  (weight ? grad_w : grad_b)[i] = s;
 }
 
 // ---------------------------------------------------------------- pilots in, grid out
@@ -1096,23 +1114,23 @@ extern "C" int hpx_conv1d_wgrad(const uint16_t* dz, const uint16_t* in, int64_t 
   const dim3 g(static_cast<unsigned>(chunks), static_cast<unsigned>((cout + 31) / 32),
                static_cast<unsigned>((taps * cin + 63) / 64));
   // Matrix-core form where the operands are whole 16-byte vectors and whole 32-channel tiles; it
-  // is the faster one for every such size, the VALU form serves the others.
+  // is the faster one for every such size, the VALU form serves the others, with the same bits.
   const bool aligned = ((reinterpret_cast<uintptr_t>(dz) | reinterpret_cast<uintptr_t>(in)) & 15u) == 0;
   if (aligned && cout % 32 == 0 && cin % 8 == 0 && cin <= 64) {
-    const int col_groups = (taps * cin + 1 + 32 * kWgWaves - 1) / (32 * kWgWaves);
-#define HPX_WGRAD(COT)                                                                                            \
-  hipLaunchKernelGGL((wgrad_mfma_kernel<COT>), dim3(chunks, cout / (32 * (COT)), col_groups), dim3(64 * kWgWaves), \
-                     (kPos * (wgrad_dz_stride<COT>() + wgrad_x_stride(cin)) + 4) * sizeof(uint16_t), s, dz, in,     \
-                     static_cast<int>(num_samples), cout, cin, taps, dilation, part_w, part_b)
-    if (cout % 224 == 0) HPX_WGRAD(7);
-    else if (cout % 64 == 0) HPX_WGRAD(2);
-    else HPX_WGRAD(1);
-#undef HPX_WGRAD
+    const auto launch = [&](auto kernel, int cot) {
+      const int tiles = (2 * cot * (taps * cin / 16 + 1) + 3) / 4, waves = wgrad_waves(cot);
+      hipLaunchKernelGGL(kernel, dim3(chunks, cout / (32 * cot), (tiles + waves - 1) / waves), dim3(64 * waves),
+                         kPos * (wgrad_dz_stride(cot) + 2 * kWgXStride) * sizeof(uint16_t), s, dz, in,
+                         static_cast<int>(num_samples), cout, cin, taps, dilation, part_w, part_b);
+    };
+    if (cout % 224 == 0) launch(wgrad_mfma_kernel<7>, 7);
+    else if (cout % 64 == 0) launch(wgrad_mfma_kernel<2>, 2);
+    else launch(wgrad_mfma_kernel<1>, 1);
   } else {
     hipLaunchKernelGGL(wgrad_kernel, g, dim3(256), 0, s, dz, in, static_cast<int>(num_samples), cout, cin, taps,
                        dilation, part_w, part_b);
   }
-  hipLaunchKernelGGL(reduce_parts_kernel, dim3(static_cast<unsigned>((nw + cout + 63) / 64)), dim3(256), 0, s, part_w,
+  hipLaunchKernelGGL(reduce_parts_kernel, dim3(blocks_for(nw + cout)), dim3(256), 0, s, part_w,
                      nw, part_b, static_cast<int64_t>(cout), chunks, grad_weight, grad_bias);
   return check_launch("hpx_conv1d_wgrad");
 }

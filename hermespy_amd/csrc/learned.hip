@@ -971,36 +971,39 @@ net_forward_kernel(const float2* __restrict__ grid, int num_drops, int num_rx, i
   if (ct < cout / 32) last(std::integral_constant<int, 1>{}, ct);
 }
 
-// Backward through the data: dz of the output rows [sample][position][224] -> dz of the three hidden
+// Backward through the data: dz of the output rows [sample][position][COUT] -> dz of the three hidden
 // layers' pre-activations, each the transposed convolution (flipped weights [cin][taps][cout]) times
 // GELU's derivative, rounded to bfloat16 for the next one and for the weight gradients.  The sums run
 // over taps, then channels, as the layer-by-layer convolutions' do, so every value is theirs: the output
-// rows of a sample lie in LDS whole (rows of 464 bytes, free of bank conflicts), which leaves room for
-// two samples a workgroup and two workgroups a CU.
+// rows of a sample lie in LDS whole (16 bytes behind each row: free of bank conflicts), which at 224 channels leaves
+// room for two samples a workgroup and two workgroups a CU.  COUT: 224 and 64, the widths that the layer-by-layer
+// backward convolution has (frames of 7168 and of 2048 elements).
 struct Gradients {
   const uint16_t* wt[3];  // transposed weights of layers 2, 3, 4
   const float* pre[3];
   uint16_t* dz[3];
 };
-constexpr int kOutChannels = 224, kOutRow = kOutChannels + 8;
 
+template <int COUT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 net_backward_kernel(const uint16_t* __restrict__ dz_out, int64_t num_samples, Gradients net) {
-  constexpr int kGroup = 2, kChunks = (kOutChannels + 63) / 64;
+  constexpr int kGroup = 2, kOutRow = COUT + 8, kFull = COUT / 64;
+  constexpr bool kHalf = COUT % 64 == 32;
+  static_assert(kHalf || COUT % 64 == 0, "whole chunks, and at most a half one");
   __shared__ __align__(16) uint16_t rows[kGroup * kPos * kOutRow];
   __shared__ __align__(16) uint16_t chunk[64 * 64];
   uint16_t* act = rows;  // the hidden rows take the output rows' place
   WeightPipe pipe{chunk, uintx4{}, uintx4{}};
-  constexpr int64_t wrow = kTaps * kOutChannels;
+  constexpr int64_t wrow = kTaps * COUT;
   pipe.fetch<64, 4>(net.wt[2], wrow);
   const int64_t s0 = static_cast<int64_t>(blockIdx.x) * kGroup;
-  constexpr int kPieces = kOutChannels / 8;
+  constexpr int kPieces = COUT / 8;
 #pragma unroll 7
   for (int i = threadIdx.x; i < kGroup * kPos * kPieces; i += 256) {
     const int row = i / kPieces, c = i - row * kPieces;  // (row: sample and position)
     const int64_t s = min(s0 + (row >> 6), num_samples - 1);
     *reinterpret_cast<uintx4*>(rows + row * kOutRow + 8 * c) =
-        *reinterpret_cast<const uintx4*>(dz_out + (s * kPos + (row & 63)) * kOutChannels + 8 * c);
+        *reinterpret_cast<const uintx4*>(dz_out + (s * kPos + (row & 63)) * COUT + 8 * c);
   }
   const TileLane ln;
   const int g = ln.sample<1>(0), half = ln.half<1>(0);
@@ -1015,23 +1018,28 @@ net_backward_kernel(const uint16_t* __restrict__ dz_out, int64_t num_samples, Gr
         acc[c][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pipe.fragment(c, j, ln), v, acc[c][0], 0, 0, 0);
     }
   };
-  static_assert(kOutChannels % 64 == 32, "whole chunks and a half one");
 #pragma unroll 1
   for (int k = 0; k < kTaps; ++k) {
-    const uint16_t* w = net.wt[2] + k * kOutChannels;
+    const uint16_t* w = net.wt[2] + k * COUT;
     const int row = ((ln.m + (k - kTaps / 2) * kDil4) & (kPos - 1)) ^ (32 * half);
     const uint16_t* a = rows + (g * kPos + row) * kOutRow + 8 * ln.kq;
+    auto next_tap = [&]() __attribute__((always_inline)) {
+      if (k + 1 < kTaps) pipe.fetch<64, 4>(w + COUT, wrow);
+      else pipe.fetch<64, 4>(net.wt[1], kTaps * 64);
+    };
 #pragma unroll
-    for (int q = 0; q + 1 < kChunks; ++q) {
+    for (int q = 0; q < kFull; ++q) {
       pipe.commit<64, 4>();
-      if (q + 2 < kChunks) pipe.fetch<64, 4>(w + 64 * (q + 1), wrow);
-      else pipe.fetch<64, 2>(w + 64 * (q + 1), wrow);
+      if (q + 1 < kFull) pipe.fetch<64, 4>(w + 64 * (q + 1), wrow);
+      else if constexpr (kHalf) pipe.fetch<64, 2>(w + 64 * kFull, wrow);
+      else next_tap();
       steps(a + 64 * q, std::integral_constant<int, 4>{});
     }
-    pipe.commit<64, 2>();
-    if (k + 1 < kTaps) pipe.fetch<64, 4>(w + kOutChannels, wrow);
-    else pipe.fetch<64, 4>(net.wt[1], kTaps * 64);
-    steps(a + 64 * (kChunks - 1), std::integral_constant<int, 2>{});
+    if constexpr (kHalf) {
+      pipe.commit<64, 2>();
+      next_tap();
+      steps(a + 64 * kFull, std::integral_constant<int, 2>{});
+    }
   }
   __syncthreads();
   auto gradient = [&](int layer) __attribute__((always_inline)) {
@@ -1274,8 +1282,8 @@ extern "C" int hpx_net_forward(const uint16_t* x, int64_t num_samples, const uin
 extern "C" int hpx_net_backward(const uint16_t* dz_out, int64_t num_samples, int cout, const uint16_t* const* weights_transposed,
                                 const float* const* pre, uint16_t* const* dz, void* stream) {
   HPX_REQUIRE(num_samples >= 0 && num_samples <= 0x7fffffff, "hpx_net_backward: invalid sample count");
-  if (cout != kOutChannels) {  // (the shape the layer-by-layer backward convolution has)
-    set_error("hpx_net_backward: cout %d not instantiated (224)", cout);
+  if (cout != 64 && cout != 224) {  // (as the layer-by-layer backward convolution)
+    set_error("hpx_net_backward: cout %d not instantiated (64, 224)", cout);
     return HPX_ERR_UNSUPPORTED;
   }
   if (num_samples == 0) return HPX_OK;
@@ -1290,7 +1298,7 @@ extern "C" int hpx_net_backward(const uint16_t* dz_out, int64_t num_samples, int
     all |= reinterpret_cast<uintptr_t>(net.wt[i]) | reinterpret_cast<uintptr_t>(pre[i]) | reinterpret_cast<uintptr_t>(dz[i]);
   }
   HPX_REQUIRE((all & 15u) == 0, "hpx_net_backward: arrays must be 16-byte aligned");
-  hipLaunchKernelGGL(net_backward_kernel, dim3(static_cast<unsigned>((num_samples + 1) / 2)), dim3(256), 0,
+  hipLaunchKernelGGL(cout == 64 ? net_backward_kernel<64> : net_backward_kernel<224>, dim3(static_cast<unsigned>((num_samples + 1) / 2)), dim3(256), 0,
                      as_stream(stream), dz_out, num_samples, net);
   return check_launch("hpx_net_backward");
 }

@@ -442,7 +442,7 @@ int hpx_nmse_grad_bf16(const float* out, const hpx_c64* csi, const hpx_c64* spat
 int hpx_net_forward(const uint16_t* x, int64_t num_samples, const uint16_t* const* weights, const float* const* biases,
                     int cout, float* const* pre, uint16_t* const* act, float* out, void* stream);
 
-/* Backward through the data in one launch: dz_out [num_samples][64][cout] (cout = 224) -> dz[i]
+/* Backward through the data in one launch: dz_out [num_samples][64][cout] (cout 64 or 224) -> dz[i]
  * [num_samples][64][64], the gradients of the hidden layers' pre-activations pre[i];
  * weights_transposed: layers 2, 3, 4 as hpx_conv1d_weight_copies writes them.  Arrays are 16-byte aligned. */
 int hpx_net_backward(const uint16_t* dz_out, int64_t num_samples, int cout, const uint16_t* const* weights_transposed,

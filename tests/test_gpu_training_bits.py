@@ -101,7 +101,8 @@ def _config(words, n):
 
 # one and two tiles of positions per wavefront (fewer than 2048 samples and more)
 @pytest.mark.parametrize("drops", [33, 520])
-@pytest.mark.parametrize("words,n", [(14, 512)])
+# 224 and 64 output channels
+@pytest.mark.parametrize("words,n", [(14, 512), (4, 512), (16, 128)])
 def test_training_step(cuda, drops, words, n):
     """Two Adam steps: activations, gradients and parameters are those of the layer-by-layer step; the loss, a float64
     sum of per-sample terms in the order their atomics arrive, is within 4096 roundings of it."""

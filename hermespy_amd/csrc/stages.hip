@@ -726,10 +726,11 @@ extern "C" int hpx_spatial_detector_host(int num_rx, int num_tx, const hpx_c128*
 
 // ------------------------------------------------------------------ random streams
 // 16 bits per thread, stored as one 16-byte piece (eight threads draw the same Philox call; one thread per call
-// storing its 128 bytes one by one took 18 us for any frame, latency alone: 2.6 us now for 86016 bits).
+// storing its 128 bytes one by one took 18 us for any frame, latency alone: 2.6 us now for 86016 bits).  `first`:
+// the first bit of the launch, a multiple of 128.
 __global__ void __launch_bounds__(256) stream_bits_kernel(uint64_t seed, uint32_t drop, uint32_t stream_id,
-                                                          int64_t nbits, uint8_t* __restrict__ bits) {
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 16;
+                                                          int64_t first, int64_t nbits, uint8_t* __restrict__ bits) {
+  const int64_t i = first + (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 16;
   if (i >= nbits) return;
   const uint4 w = stream_call(seed, drop, stream_id, static_cast<uint32_t>(i >> 7));
   const int k = static_cast<int>(i >> 5) & 3;
@@ -748,9 +749,13 @@ extern "C" int hpx_stream_bits(uint64_t seed, uint32_t drop, uint32_t stream_id,
   HPX_REQUIRE(num_bits >= 0 && num_bits <= (int64_t(1) << 38), "hpx_stream_bits: invalid length");
   if (num_bits == 0) return HPX_OK;
   HPX_REQUIRE(bits, "hpx_stream_bits: null pointer");
-  const int64_t pieces = (num_bits + 15) / 16;
-  hipLaunchKernelGGL(stream_bits_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
-                     HPX_STREAM(stream), seed, drop, stream_id, num_bits, bits);
+  // (a launch holds fewer than 2^32 threads)
+  constexpr int64_t kLaunchBits = int64_t(1) << 35;
+  for (int64_t first = 0; first < num_bits; first += kLaunchBits) {
+    const int64_t pieces = (std::min(num_bits - first, kLaunchBits) + 15) / 16;
+    hipLaunchKernelGGL(stream_bits_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
+                       HPX_STREAM(stream), seed, drop, stream_id, first, num_bits, bits);
+  }
   return check_launch("hpx_stream_bits");
 }
 

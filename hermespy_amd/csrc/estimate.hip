@@ -53,6 +53,7 @@ constexpr int kGemmRows = 64, kGemmCols = 128, kGemmK = 32;
 constexpr int kGemmStride = kGemmK + 2;  // float2; rows 16 bytes apart modulo the LDS banks
 constexpr int kGemmSets = 16;            // filter sets per launch
 constexpr int kXcds = 8;                 // consecutive workgroups go round robin over the XCDs
+constexpr int kGemmTiles = (1 << 24) - kXcds;  // tiles per launch: fewer than 2^32 threads
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
@@ -62,6 +63,7 @@ struct LmmseSets {
   int count[kGemmSets];
   int first_tile[kGemmSets + 1];
   int num_sets;
+  int begin, end;  // this launch's tiles
 };
 
 // VEC: the rows of ls and of the filters are whole 16-byte vectors.
@@ -72,10 +74,9 @@ lmmse_kernel(LmmseSets sets, const float2* __restrict__ ls, int64_t ls_tx_stride
                                                     int col_tiles, float2* __restrict__ est, int64_t est_tx_stride) {
   __shared__ __align__(16) float2 as[kGemmRows * kGemmStride];
   __shared__ __align__(16) float2 bs[kGemmCols * kGemmStride];
-  const int total = sets.first_tile[sets.num_sets];
-  const int per_xcd = (total + kXcds - 1) / kXcds;
-  const int tile = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
-  if (tile >= total) return;
+  const int per_xcd = (sets.end - sets.begin + kXcds - 1) / kXcds;
+  const int tile = sets.begin + static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
+  if (tile >= sets.end) return;
   int si = 0;
   while (tile >= sets.first_tile[si + 1]) ++si;
   const int count = sets.count[si];
@@ -327,14 +328,19 @@ int lmmse_launch(const char* what, const hpx_c64* ls, int num_tx, int64_t num_ro
                  int64_t set_stride, int64_t elements, const void* const* rows, const int* counts, int num_sets,
                  hpx_c64* est, void* stream) {
   const int64_t col_tiles = (elements + kGemmCols - 1) / kGemmCols;
+  HPX_REQUIRE(col_tiles <= 65535, "%s: grid too large", what);
   const bool vec = num_pilots % 2 == 0 &&
                    ((reinterpret_cast<uintptr_t>(ls) | reinterpret_cast<uintptr_t>(filters)) & 15u) == 0;
   auto flush = [&](LmmseSets& sets) -> int {
     if (sets.num_sets == 0) return HPX_OK;
-    const unsigned blocks = static_cast<unsigned>((sets.first_tile[sets.num_sets] + kXcds - 1) / kXcds * kXcds);
-    hipLaunchKernelGGL(vec ? lmmse_kernel<true> : lmmse_kernel<false>, dim3(blocks), dim3(256), 0, as_stream(stream), sets,
-                       reinterpret_cast<const float2*>(ls), num_rows * num_pilots, num_pilots, elements * num_pilots,
-                       elements, static_cast<int>(col_tiles), reinterpret_cast<float2*>(est), num_rows * elements);
+    const int total = sets.first_tile[sets.num_sets];
+    for (sets.begin = 0; sets.begin < total; sets.begin = sets.end) {
+      sets.end = std::min(total, sets.begin + kGemmTiles);
+      const unsigned blocks = static_cast<unsigned>((sets.end - sets.begin + kXcds - 1) / kXcds * kXcds);
+      hipLaunchKernelGGL(vec ? lmmse_kernel<true> : lmmse_kernel<false>, dim3(blocks), dim3(256), 0, as_stream(stream), sets,
+                         reinterpret_cast<const float2*>(ls), num_rows * num_pilots, num_pilots, elements * num_pilots,
+                         elements, static_cast<int>(col_tiles), reinterpret_cast<float2*>(est), num_rows * elements);
+    }
     sets.num_sets = 0;
     return check_launch(what);
   };

@@ -27,3 +27,24 @@ def test_stream_bits(cuda):
         want = ((words[:, None] >> np.arange(32, dtype=np.uint32)) & 1).reshape(-1).astype(np.uint8)
         got = bits[first:first + 128].cpu().numpy()
         assert np.array_equal(got, want[:got.size])
+
+
+def test_lmmse_rows(cuda):
+    """2^24 tiles of 64 rows, one pilot and one element: every row is the product of its value and the filter's (a
+    complex product in float32: each part within two roundings of its terms)."""
+
+    from hermespy_amd import _lib
+
+    rows, nt = 1 << 28, 4
+    g = torch.Generator(device=cuda).manual_seed(9)
+    ls = torch.view_as_complex(torch.randn(nt, rows, 2, generator=g, device=cuda))
+    filt = torch.view_as_complex(torch.randn(nt, 1, 1, 2, generator=g, device=cuda))
+    index = torch.arange(rows, dtype=torch.int32, device=cuda)
+    est = torch.full((nt, rows), complex("nan"), dtype=torch.complex64, device=cuda)
+    _lib.check(_lib.load().hpx_lmmse_apply(_lib.ptr(ls), nt, rows, 1, _lib.ptr(filt), 1, _lib.ptr(index), rows, _lib.ptr(est),
+                                           _lib.stream_handle()))
+    for t in range(nt):
+        for part in range(0, rows, rows // 8):
+            x, got = ls[t, part:part + rows // 8], est[t, part:part + rows // 8]
+            error = torch.view_as_real(got - x * filt[t, 0, 0]).abs().amax(dim=-1)
+            assert bool((error <= 4 * 2.0**-24 * 2 * x.abs() * filt[t, 0, 0].abs()).all())

@@ -701,6 +701,13 @@ __device__ __forceinline__ void zero_tiles(floatx16 (&acc)[CT][PT]) {
       for (int r = 0; r < 16; ++r) acc[c][t][r] = 0.0f;
 }
 
+// Eight weights in one load, wherever they lie: the caller's weights need no more than their own alignment.
+__device__ __forceinline__ uintx4 load8(const uint16_t* p) {
+  uintx4 v;
+  __builtin_memcpy(&v, p, sizeof(v));
+  return v;
+}
+
 // Weights on their way to LDS: the workgroup loads a chunk (up to 64 output channels by 64 elements of
 // their rows, whole 128-byte lines) into registers while the chunk before it is in use, and all
 // wavefronts read their fragments from the copy in LDS, rows permuted like the activations'.  (Fragments
@@ -716,8 +723,8 @@ struct WeightPipe {
     static_assert(kTotal == 256 || kTotal == 512, "one or two whole pieces per thread");
     const int row = static_cast<int>(threadIdx.x) / kPieces, c = static_cast<int>(threadIdx.x) % kPieces;
     const uint16_t* p = w + row * wrow + 8 * c;
-    r0 = *reinterpret_cast<const uintx4*>(p);
-    if constexpr (kTotal == 512) r1 = *reinterpret_cast<const uintx4*>(p + (256 / kPieces) * wrow);
+    r0 = load8(p);
+    if constexpr (kTotal == 512) r1 = load8(p + (256 / kPieces) * wrow);
   }
   template <int ROWS, int STEPS>
   __device__ __forceinline__ void commit() {
@@ -776,7 +783,7 @@ __device__ __forceinline__ void conv_input(const uint16_t* xs, const uint16_t* _
     bf16x8 wv[CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
-      uintx4 v = *reinterpret_cast<const uintx4*>(wl + c * 32 * (TAPS * 8) + min(tap, TAPS - 1) * 8);
+      uintx4 v = load8(wl + c * 32 * (TAPS * 8) + min(tap, TAPS - 1) * 8);
       if (tap >= TAPS) v = uintx4{0u, 0u, 0u, 0u};
       wv[c] = __builtin_bit_cast(bf16x8, v);
     }

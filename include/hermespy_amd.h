@@ -423,7 +423,7 @@ int hpx_nmse_grad(const float* out, const hpx_c64* csi, const hpx_c64* spatial, 
  * biases: host arrays of 5 device pointers (layers 1-4, then the skip convolution), bfloat16
  * [cout][taps][cin] with (cin, taps) = (8, 5), (64, 5), (64, 5), (64, 5), (8, 17) and float32 [cout];
  * cout = 64 for the hidden layers and 2 words N / 64 for the last two; noise_power [num_drops] feeds
- * the SNR input channel.  Same arithmetic as hpx_net_input + hpx_conv1d_forward (x4, then mode 2)
+ * the SNR input channel.  Weights and biases need no more than their elements' alignment.  Same arithmetic as hpx_net_input + hpx_conv1d_forward (x4, then mode 2)
  * + hpx_net_output. */
 int hpx_learned_estimate(const hpx_c64* grid, int64_t num_drops, int num_rx, int num_tx, int words,
                          int num_subcarriers, const int32_t* pilot_index, const hpx_c64* pilot_values, int num_pilots,
@@ -438,7 +438,7 @@ int hpx_nmse_grad_bf16(const float* out, const hpx_c64* csi, const hpx_c64* spat
 /* Forward pass of a training step in one launch: x [num_samples][64][8] through the network of
  * hpx_learned_estimate; pre[i] / act[i] (host arrays of 3 device pointers) [num_samples][64][64] are the
  * hidden layers' pre-activations (float32) and activations (bfloat16), out [num_samples][64][cout]
- * the output.  Arrays are 16-byte aligned. */
+ * the output.  x, pre, act and out are 16-byte aligned. */
 int hpx_net_forward(const uint16_t* x, int64_t num_samples, const uint16_t* const* weights, const float* const* biases,
                     int cout, float* const* pre, uint16_t* const* act, float* out, void* stream);
 

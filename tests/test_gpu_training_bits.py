@@ -132,3 +132,43 @@ def test_training_step(cuda, drops, words, n):
             assert torch.equal(p, new)
         for w, w16 in zip(tr.net.w, tr.net.w16):
             assert torch.equal(w.to(torch.bfloat16), w16)
+
+
+# one and two tiles of positions per wavefront
+@pytest.mark.parametrize("s", [5, 2050])
+def test_weights_of_any_alignment(cuda, s):
+    """Inference and training forward read weights and biases one element off their 16-byte boundary: the same bits."""
+
+    from hermespy_amd import _lib
+
+    lib, st = _lib.load(), _lib.stream_handle()
+    g = torch.Generator(device=cuda).manual_seed(s)
+    shapes = [(64, 5, 8), (64, 5, 64), (64, 5, 64), (64, 5, 64), (64, 17, 8)]
+    w = [(torch.randn(sh, generator=g, device=cuda) * 0.1).to(torch.bfloat16) for sh in shapes]
+    b = [torch.randn(64, generator=g, device=cuda) for _ in shapes]
+    x = torch.randn(s, 64, 8, generator=g, device=cuda).to(torch.bfloat16)
+    grid = torch.view_as_complex(torch.randn(s, 4, 512, 2, generator=g, device=cuda))
+    pidx = torch.arange(0, 256, 2, dtype=torch.int32, device=cuda)
+    pval = torch.ones(128, dtype=torch.complex64, device=cuda)
+    noise = torch.ones(s, dtype=torch.float64, device=cuda)
+
+    def pointers(tensors):
+        return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+    def passes(weights, biases):
+        wp, bp = pointers(weights), pointers(biases)
+        est = torch.full((s, 4, 512), complex("nan"), dtype=torch.complex64, device=cuda)
+        _lib.check(lib.hpx_learned_estimate(grid.data_ptr(), s, 1, 1, 4, 512, pidx.data_ptr(), pval.data_ptr(), 128,
+                                            noise.data_ptr(), ctypes.addressof(wp), ctypes.addressof(bp), 64,
+                                            est.data_ptr(), st))
+        pre = [torch.empty((s, 64, 64), device=cuda) for _ in range(3)]
+        act = [torch.empty((s, 64, 64), dtype=torch.bfloat16, device=cuda) for _ in range(3)]
+        out = torch.empty((s, 64, 64), device=cuda)
+        pp, ap = pointers(pre), pointers(act)
+        _lib.check(lib.hpx_net_forward(x.data_ptr(), s, wp, bp, 64, pp, ap, out.data_ptr(), st))
+        return [est, out, *pre, *act]
+
+    shifted = [torch.cat([t.new_zeros(1), t.reshape(-1)])[1:] for t in w + b]
+    assert all(t.data_ptr() % 16 == t.element_size() for t in shifted)
+    for got, want in zip(passes(shifted[:5], shifted[5:]), passes(w, b)):
+        assert torch.equal(got, want)

@@ -566,7 +566,7 @@ __global__ void __launch_bounds__(256) loss_grad_kernel(const float* __restrict_
                                                         GRAD* __restrict__ grad) {
   const int64_t s = blockIdx.x;
   const int64_t wn = static_cast<int64_t>(words) * n;
-  const float2* row = reinterpret_cast<const float2*>(out) + s * wn;
+  const float* row = out + 2 * s * wn;  // (aligned as floats are, like the gradient)
   float2 sp;
   const float2* c = ideal_parts(csi, spatial, s, num_drops, num_rx, num_tx, wn, &sp);
   const float scale = static_cast<float>(work[2 * num_groups + sample_group(s, num_drops, num_rx, group)]);
@@ -574,12 +574,18 @@ __global__ void __launch_bounds__(256) loss_grad_kernel(const float* __restrict_
 #pragma unroll 4
   for (int i = threadIdx.x; i < wn; i += blockDim.x, at.next()) {
     const float2 h = cmul(sp, c[at.element(n)]);
-    const float2 v = row[i];
-    const float gr = scale * (v.x - h.x), gi = scale * (v.y - h.y);
-    if constexpr (sizeof(GRAD) == 2)
-      reinterpret_cast<uint32_t*>(grad)[s * wn + i] = f2bf(gr) | static_cast<uint32_t>(f2bf(gi)) << 16;
-    else
-      reinterpret_cast<float2*>(grad)[s * wn + i] = make_float2(gr, gi);
+    float v[2];
+    __builtin_memcpy(v, row + 2 * i, sizeof(v));
+    const float gr = scale * (v[0] - h.x), gi = scale * (v[1] - h.y);
+    GRAD pair[2];
+    if constexpr (sizeof(GRAD) == 2) {
+      pair[0] = f2bf(gr);
+      pair[1] = f2bf(gi);
+    } else {
+      pair[0] = gr;
+      pair[1] = gi;
+    }
+    __builtin_memcpy(grad + 2 * (s * wn + i), pair, sizeof(pair));
   }
 }
 

@@ -172,3 +172,34 @@ def test_weights_of_any_alignment(cuda, s):
     assert all(t.data_ptr() % 16 == t.element_size() for t in shifted)
     for got, want in zip(passes(shifted[:5], shifted[5:]), passes(w, b)):
         assert torch.equal(got, want)
+
+
+# one workgroup per sample, and samples in shares (a pair or none for the last threads)
+@pytest.mark.parametrize("drops,words,n", [(1, 14, 4096), (3, 3, 192), (1100, 1, 64)])
+def test_loss_gradient_of_any_alignment(cuda, drops, words, n):
+    """Outputs and gradients one element off the boundary of a pair: the bits of aligned ones, float32 and bfloat16,
+    which for one group are scale (out - H)."""
+
+    from hermespy_amd import _lib
+
+    lib, st = _lib.load(), _lib.stream_handle()
+    g = torch.Generator(device=cuda).manual_seed(n)
+    blk = n // 64
+    out = torch.randn(drops, 64, words, blk, 2, generator=g, device=cuda)
+    csi = torch.view_as_complex(torch.randn(drops, words, n, 2, generator=g, device=cuda))
+    spatial = torch.ones(drops, 1, 1, dtype=torch.complex64, device=cuda)
+
+    def gradient(fn, dtype, offset):
+        flat = torch.full((out.numel() + offset,), float("nan"), dtype=dtype, device=cuda)
+        src = torch.cat([out.new_zeros(offset), out.reshape(-1)])
+        work = torch.zeros(3, dtype=torch.float64, device=cuda)
+        loss = torch.zeros(1, dtype=torch.float64, device=cuda)
+        _lib.check(fn(src[offset:].data_ptr(), csi.data_ptr(), spatial.data_ptr(), drops, 1, 1, words, n, None, 1,
+                      work.data_ptr(), flat[offset:].data_ptr(), loss.data_ptr(), st))
+        return flat[offset:], work
+
+    got, work = gradient(lib.hpx_nmse_grad, torch.float32, 1)
+    h = torch.view_as_real(csi).reshape(drops, words, 64, blk, 2).permute(0, 2, 1, 3, 4)
+    assert torch.equal(got, (work[2].float() * (out - h)).reshape(-1))
+    assert torch.equal(gradient(lib.hpx_nmse_grad_bf16, torch.bfloat16, 1)[0], got.to(torch.bfloat16))
+    assert torch.equal(gradient(lib.hpx_nmse_grad, torch.float32, 0)[0], got)

@@ -557,7 +557,7 @@ __global__ void loss_finish_kernel(int num_groups, double* __restrict__ work, do
   loss[0] = used ? l / used : 0.0;
 }
 
-// One workgroup per sample; GRAD: float, or bfloat16 (uint16_t) for the backward pass.
+// Workgroup (sample, share of its pairs); GRAD: float, or bfloat16 (uint16_t) for the backward pass.
 template <class GRAD>
 __global__ void __launch_bounds__(256) loss_grad_kernel(const float* __restrict__ out, const float2* __restrict__ csi,
                                                         const float2* __restrict__ spatial, int num_drops, int num_rx,
@@ -570,9 +570,11 @@ __global__ void __launch_bounds__(256) loss_grad_kernel(const float* __restrict_
   float2 sp;
   const float2* c = ideal_parts(csi, spatial, s, num_drops, num_rx, num_tx, wn, &sp);
   const float scale = static_cast<float>(work[2 * num_groups + sample_group(s, num_drops, num_rx, group)]);
-  PairWalk at(threadIdx.x, blockDim.x, words, n);
+  const int first = static_cast<int>(blockIdx.y * blockDim.x + threadIdx.x);
+  const int step = static_cast<int>(gridDim.y * blockDim.x);
+  PairWalk at(first, step, words, n);
 #pragma unroll 4
-  for (int i = threadIdx.x; i < wn; i += blockDim.x, at.next()) {
+  for (int i = first; i < wn; i += step, at.next()) {
     const float2 h = cmul(sp, c[at.element(n)]);
     float v[2];
     __builtin_memcpy(v, row + 2 * i, sizeof(v));
@@ -1235,7 +1237,13 @@ int nmse_grad(const char* name, const float* out, const hpx_c64* csi, const hpx_
   hipLaunchKernelGGL(loss_accumulate_kernel, g, dim3(256), 0, s, out, c, sp, nd, num_rx, num_tx, words, num_subcarriers,
                      group, num_groups, work);
   hipLaunchKernelGGL(loss_finish_kernel, dim3(1), dim3(64), 0, s, num_groups, work, loss);
-  hipLaunchKernelGGL((loss_grad_kernel<GRAD>), g, dim3(256), 0, s, out, c, sp, nd, num_rx, num_tx, words, num_subcarriers,
+  // Few samples in shares, up to 1024 workgroups (four a CU): the whole call with one sample of 57344 pairs 103 us in
+  // one workgroup, 61 in shares, with 16 of 573440 1679 and 939 us; from 1024 samples on each is one share.  A sample
+  // of 64 pairs is one wavefront.
+  const int64_t pairs = static_cast<int64_t>(words) * num_subcarriers;
+  const int64_t threads = std::min<int64_t>(256, (pairs + 63) / 64 * 64);
+  const dim3 gs(g.x, static_cast<unsigned>(std::max<int64_t>(1, std::min((pairs + threads - 1) / threads, 1024 / samples))));
+  hipLaunchKernelGGL((loss_grad_kernel<GRAD>), gs, dim3(static_cast<unsigned>(threads)), 0, s, out, c, sp, nd, num_rx, num_tx, words, num_subcarriers,
                      group, num_groups, work, grad);
   return check_launch(name);
 }

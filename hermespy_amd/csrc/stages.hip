@@ -517,6 +517,7 @@ constexpr int kCsiThreads = 256;
 // kCsiTerms) a thread does its path's terms one after the other.  16 paths of 21 terms at 1024 subcarriers
 // and 14 words: 34 us with the terms in turn and a workgroup per word, 9.4 us now.
 constexpr int kCsiTerms = 1536;  // (path, term) pairs: 36 KB
+constexpr int kCsiGroups = 1024;  // workgroups up to which words are cut into shares
 
 template <bool TERMS>
 __global__ void __launch_bounds__(kCsiThreads) ideal_csi_kernel(const double* __restrict__ sos, int paths, int terms,
@@ -593,7 +594,10 @@ extern "C" int hpx_ideal_csi(const double* sos, int num_paths, int num_terms, co
   const bool by_term = static_cast<int64_t>(num_paths) * num_terms <= kCsiTerms &&
                        lds + 3 * sizeof(double) * num_paths * num_terms <= 64 * 1024;
   if (by_term) lds += 3 * sizeof(double) * num_paths * num_terms;
-  const dim3 g(static_cast<unsigned>(words), static_cast<unsigned>((num_subcarriers + kCsiThreads - 1) / kCsiThreads));
+  // A share computes its word's means and twiddles anew, so words are cut only while the launch leaves the GPU room:
+  // 4096 subcarriers and 100 paths of 21 terms, 14 words 162 us whole and 31 in 16 shares each, 1400 words 364 and 801.
+  const int shares = std::max(1, std::min((num_subcarriers + kCsiThreads - 1) / kCsiThreads, kCsiGroups / words));
+  const dim3 g(static_cast<unsigned>(words), static_cast<unsigned>(shares));
   hipLaunchKernelGGL(by_term ? ideal_csi_kernel<true> : ideal_csi_kernel<false>, g, dim3(kCsiThreads), lds,
                      HPX_STREAM(stream), sos, num_paths, num_terms, delays, keep_below,
                      reinterpret_cast<const float2*>(spatial), num_rx, num_tx, words, num_subcarriers, prefix,

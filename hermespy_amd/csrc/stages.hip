@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(kTdlThreads) tdl_propagate_kernel(
   extern __shared__ float2 coeff[];  // [paths][nb][kTaylorCoeffs], STAGE: after the window [ntx][kTdlThreads + max_delay]
   const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kTdlThreads;
   const int64_t out_len = m_len + max_delay;
-  const int width = kTdlThreads + max_delay;
+  const int width = STAGE ? kTdlThreads + max_delay : 0;
   const float2* window = coeff;
   float2* const coef = coeff + (STAGE ? ntx * width : 0);
   if constexpr (STAGE) {
@@ -171,6 +171,18 @@ __global__ void __launch_bounds__(kTdlThreads) tdl_propagate_kernel(
   }
 }
 
+// Whether the window goes through LDS: it is read once and waited for before the first path, which pays where the
+// paths read every sample of it several times.  With few workgroups (latency) a thread's reads have to be many;
+// with many (throughput) little reuse is enough while the window leaves the CU several workgroups.  Times in us
+// through memory and through LDS, antennas / paths / max delay / samples: 1/1/6000/2M 48 and 143, 2/3/2000/2M 67 and 128,
+// 4/3/20/100K 13.0 and 14.0, 4/3/20/2M 83 and 72, 4/8/1000/2M 131 and 214, 4/23/300/500K 76 and 49,
+// 8/5/300/2M 154 and 187, 8/23/300/2M 400 and 276, 4/8/20/500K 34 and 30, 1/23/300/100K 16.6 and 16.2.
+bool stage_window(int64_t groups, int num_tx, int paths, int64_t width, int64_t bytes) {
+  const double reuse = static_cast<double>(paths) * kTdlThreads / static_cast<double>(width);
+  if (groups >= 4096) return reuse >= 6.0 || (reuse >= 1.3 && bytes <= 20 * 1024);
+  return reuse >= 3.5 && static_cast<int64_t>(paths) * num_tx >= (groups >= 1024 ? 12 : 32);
+}
+
 extern "C" int hpx_tdl_propagate(const hpx_c64* x, int num_tx, int64_t ld_x, int64_t num_samples, const double* sos,
                                  int num_paths, int num_terms, double max_abs_rate, const int32_t* delays,
                                  int32_t max_delay, const hpx_c64* spatial, int num_rx, hpx_c64* y, int64_t ld_y,
@@ -196,8 +208,9 @@ extern "C" int hpx_tdl_propagate(const hpx_c64* x, int num_tx, int64_t ld_x, int
     }
   }
   const dim3 grid(static_cast<unsigned>((out_len + kTdlThreads - 1) / kTdlThreads));
-  const int64_t window = (static_cast<int64_t>(kTdlThreads) + max_delay) * num_tx * static_cast<int64_t>(sizeof(float2));
-  const bool stage = static_cast<int64_t>(lds) + window <= 64 * 1024;
+  const int64_t width = static_cast<int64_t>(kTdlThreads) + max_delay;
+  const int64_t window = width * num_tx * static_cast<int64_t>(sizeof(float2));
+  const bool stage = static_cast<int64_t>(lds) + window <= 64 * 1024 && stage_window(grid.x, num_tx, num_paths, width, window);
   if (stage) lds += static_cast<size_t>(window);
   hipLaunchKernelGGL(stage ? tdl_propagate_kernel<true> : tdl_propagate_kernel<false>, grid, dim3(kTdlThreads), lds, HPX_STREAM(stream),
                      reinterpret_cast<const float2*>(x), num_tx, ld_x, num_samples, sos, num_paths, num_terms, log2b,

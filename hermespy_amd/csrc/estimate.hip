@@ -10,6 +10,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <array>
 
 #include "hpx_common.hpp"
 #include "hpx_detect.hpp"
@@ -290,21 +291,40 @@ __global__ void __launch_bounds__(256) zero_counts_kernel(int32_t* __restrict__ 
 // latency and takes shares up to 4096 workgroups; one that streams from HBM only two workgroups a CU, at least
 // one a drop: a 2x2 512-subcarrier link with one and with more shares, 11 drops 63 and 15 us, 400 (183 MB)
 // 55 and 34, 600 (275 MB) 73 and 51, 1000 (459 MB) 102 and 109.  The line lies between the last two.
-int detect_segments(int64_t drops, int64_t drop_bytes, int words) {
+// A share has at least a workgroup's threads of elements, and drops of a few steps are not cut: 200 drops of 14
+// words of 64 subcarriers, one stream 7.7 us with a workgroup a drop, 12.5 in 14 shares each, 5.3 whole; two streams 11.7,
+// 13.9 and in four shares 8.8; eight streams 59, 72 and 35.
+int detect_segments(int64_t drops, int64_t drop_bytes, int words, int64_t elements, int streams) {
+  if (elements * streams <= 1024) return 1;
   const int64_t target = drops * drop_bytes <= (int64_t(384) << 20) ? 4096 : 512;
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(words, target / std::max<int64_t>(drops, 1))));
+  const int64_t most = std::min<int64_t>(words, (elements + 255) / 256);
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(most, target / std::max<int64_t>(drops, 1))));
+}
+
+// The boundaries of the four constellations, found once (500 steps of a bisection: a tenth of a small call).
+const DemapBounds& bounds_of(const Modulation& mod) {
+  static const auto all = [] {
+    std::array<DemapBounds, 4> b{};
+    for (int i = 0; i < 4; ++i) {
+      Modulation m;
+      if (modulation(4 << (2 * i), 1, &m)) b[i] = demap_bounds(m);
+    }
+    return b;
+  }();
+  return all[mod.bps / 2 - 1];
 }
 
 template <int NT>
 int detect_launch(const Modulation& mod, const float2* grid, const float2* est, int num_drops, int num_rx, int words, int n,
                   const int32_t* elements, const int32_t* word_data, int mmse, const double* noise_power, uint64_t seed,
                   int64_t first_drop, int data_total, int32_t* errors, float2* equalized, hipStream_t stream) {
-  const int segs = detect_segments(num_drops, 8 * static_cast<int64_t>(words) * n * (num_rx + num_rx * NT + NT), words);
+  const int64_t per_drop = static_cast<int64_t>(words) * n;
+  const int segs = detect_segments(num_drops, 8 * per_drop * (num_rx + num_rx * NT + NT), words, per_drop, NT);
   // (a share holds at most this many bits a stream, and begins inside a call)
   const int64_t share = static_cast<int64_t>((words + segs - 1) / segs) * n * mod.bps;
   const int64_t want = 4 * ((share + 127) / 128 + 1);
   const int bits_words = want * NT * 4 <= 48 * 1024 ? static_cast<int>(want) : 0;
-  const DemapBounds bounds = demap_bounds(mod);
+  const DemapBounds& bounds = bounds_of(mod);
   if (segs > 1)
     hipLaunchKernelGGL(zero_counts_kernel, dim3(static_cast<unsigned>((num_drops + 255) / 256)), dim3(256), 0, stream, errors,
                        num_drops);

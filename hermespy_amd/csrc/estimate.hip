@@ -48,8 +48,10 @@ __global__ void __launch_bounds__(256) pilot_ls_kernel(const float2* __restrict_
 // loads in flight; a lane's 16-byte LDS read holds two pilots, which feed 16 MFMAs per three reads.
 // All sets go in one launch (a set alone is a few hundred workgroups), with the row tiles of one
 // filter tile next to each other on one XCD, whose L2 then serves the filter.  Bound: float32 MFMA.
-// 1000 drops of the 2x2 512-subcarrier link at 11 SNR points (29.4 GFLOP, 0.39 GB): 283 us,
-// 104 TFLOP/s (a 32 x 128 FP32 VALU tile and a launch per SNR point took 741 us).
+// 1000 drops of the 2x2 512-subcarrier link at 11 SNR points (29.4 GFLOP, 0.39 GB): 278 us,
+// 106 TFLOP/s (a 32 x 128 FP32 VALU tile and a launch per SNR point took 741 us).  Small calls are latency: the
+// contraction's padding and an empty upper half of the rows are left out (one row of 128 pilots and 7168 elements,
+// 2 streams: 21.9 us with them, 14.8 without; 100 rows of 16 pilots and 64 elements 12.3 and 7.3, with the VALU tile 9.5).
 constexpr int kGemmRows = 64, kGemmCols = 128, kGemmK = 32;
 constexpr int kGemmStride = kGemmK + 2;  // float2; rows 16 bytes apart modulo the LDS banks
 constexpr int kGemmSets = 16;            // filter sets per launch
@@ -75,6 +77,7 @@ lmmse_kernel(LmmseSets sets, const float2* __restrict__ ls, int64_t ls_tx_stride
                                                     int col_tiles, float2* __restrict__ est, int64_t est_tx_stride) {
   __shared__ __align__(16) float2 as[kGemmRows * kGemmStride];
   __shared__ __align__(16) float2 bs[kGemmCols * kGemmStride];
+  __shared__ int32_t row_of[kGemmRows];  // for the stores (read before the first barrier, not after the last)
   const int per_xcd = (sets.end - sets.begin + kXcds - 1) / kXcds;
   const int tile = sets.begin + static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
   if (tile >= sets.end) return;
@@ -107,6 +110,8 @@ lmmse_kernel(LmmseSets sets, const float2* __restrict__ ls, int64_t ls_tx_stride
     const int64_t e = e0 + sr + 16 * i;
     brow[i] = ft + (e < elements ? e : elements - 1) * num_pilots;
   }
+  if (tid < kGemmRows && r0 + tid < count) row_of[tid] = rows[r0 + tid];
+  const bool upper = r0 + 32 < count;  // rows in the upper half of the tile
   floatx4 ra[kA], rb[kB];
   auto pair_at = [&](const float2* row, int k) __attribute__((always_inline)) {
     floatx4 v = {0.f, 0.f, 0.f, 0.f};
@@ -146,20 +151,23 @@ lmmse_kernel(LmmseSets sets, const float2* __restrict__ ls, int64_t ls_tx_stride
     if (k0 + kGemmK < num_pilots) load(k0 + kGemmK);
 #pragma unroll
     for (int s = 0; s < kGemmK / 4; ++s) {
+      if (k0 + 4 * s >= num_pilots) break;  // (padding)
       const floatx4 b = *reinterpret_cast<const floatx4*>(bs + (32 * wave + mrow) * kGemmStride + 4 * s + 2 * kq);
       floatx4 a[2];
 #pragma unroll
       for (int m = 0; m < 2; ++m)
         a[m] = *reinterpret_cast<const floatx4*>(as + (32 * m + mrow) * kGemmStride + 4 * s + 2 * kq);
 #pragma unroll
-      for (int o = 0; o < 4; o += 2)
+      for (int m = 0; m < 2; ++m) {
+        if (m && !upper) break;
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
+        for (int o = 0; o < 4; o += 2) {
           re[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[m][o], b[o], re[m], 0, 0, 0);
           im[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[m][o], b[o + 1], im[m], 0, 0, 0);
           re[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(-a[m][o + 1], b[o + 1], re[m], 0, 0, 0);
           im[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[m][o + 1], b[o], im[m], 0, 0, 0);
         }
+      }
     }
     __syncthreads();
   }
@@ -170,8 +178,8 @@ lmmse_kernel(LmmseSets sets, const float2* __restrict__ ls, int64_t ls_tx_stride
   for (int m = 0; m < 2; ++m)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = r0 + 32 * m + 8 * (r >> 2) + 4 * kq + (r & 3);
-      if (row < count) et[static_cast<int64_t>(rows[row]) * elements + e] = make_float2(re[m][r], im[m][r]);
+      const int row = 32 * m + 8 * (r >> 2) + 4 * kq + (r & 3);
+      if (r0 + row < count) et[static_cast<int64_t>(row_of[row]) * elements + e] = make_float2(re[m][r], im[m][r]);
     }
 }
 

@@ -575,7 +575,7 @@ extern "C" int hpx_run_batch_drops(const hpx_link* link_host, const hpx_frame* f
 // path (frame / 64 + 16) x terms sines and cosines instead of frame x terms, and per 8 samples and
 // term one complex product and 8 multiply-adds on table entries that LDS broadcasts.  Every phase
 // is a product w x samples near zero, which costs less rounding than a direct evaluation's
-// w x samples + phi; the products add about as much back.  The OFDM transforms are radix-4 Stockham passes over the whole
+// w x samples + phi, and the products add about as much back: the error is about the same.  The OFDM transforms are radix-4 Stockham passes over the whole
 // frame between the two signal buffers (less rounding than the direct sums they replace).  The
 // tables and the prologue's uniforms live in the receive buffer, which is empty until the channel's
 // outputs leave their registers, so four drops share a CU.  5000 drops of 64 subcarriers, 5 paths:
@@ -587,10 +587,12 @@ constexpr int kF64MaxSubcarriers = 256;
 constexpr int kF64Run = 8;       // consecutive output samples per thread
 constexpr int kF64Block = 64;    // samples per first factor of the phase
 constexpr int kF64Round = kF64Run * kF64Threads;  // output samples per round of the workgroup
+constexpr int kF64Tables = 512;  // complex128 values the tables may take beyond a short frame's
 
 struct F64Layout {
   int off_sos, off_tw, off_x, off_y, off_abar, off_bits, off_red;
   int dx, frame, bits_words;
+  int work;        // complex128 values of the receive buffer: the frame, or more for the sinusoids' tables
   int term_group;  // sinusoids whose tables fit the receive buffer at once
   int64_t bytes;
 };
@@ -667,6 +669,10 @@ __device__ __forceinline__ void f64_fft(const double2* src, int sstride, double2
   }
 }
 
+// RUN: output samples per thread of the channel, consecutive: kF64Run, or one for frames of at most a workgroup's threads,
+// whose few runs of eight would be one long chain (the same products and sums per sample): one drop of a word of 32
+// subcarriers and 15 paths 119 us in runs of eight, 59 in single samples, 109 with a sine and cosine per sample.
+template <int RUN>
 __global__ void __launch_bounds__(kF64Threads) __attribute__((amdgpu_waves_per_eu(4)))
 f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
   extern __shared__ __align__(16) unsigned char lds[];
@@ -729,7 +735,7 @@ f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
       row[0] = rate;
       row[1] = amp * cs;
       row[2] = amp * sn;
-      if (e < g.frame * 2) dir[e] = dirichlet_factor(rate, n);
+      if (e < g.work * 2) dir[e] = dirichlet_factor(rate, n);
     }
   }
   // spatial response of the single antenna pair: exp(2 pi j u_00) (fading.py:476-489)
@@ -747,7 +753,7 @@ f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
         for (int k = tid & 3; k < terms; k += 4) {
           const int i = p * terms + k;
           const double rate = sos[3 * i];
-          const double wgt = i < g.frame * 2 ? dir[i] : dirichlet_factor(rate, n);
+          const double wgt = i < g.work * 2 ? dir[i] : dirichlet_factor(rate, n);
           double s, c;
           sincos(reduce_phase(rate * centre), &s, &c);
           const double2 v = dcmul(make_double2(sos[3 * i + 1], sos[3 * i + 2]), make_double2(c, s));
@@ -788,17 +794,17 @@ f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
   const double sigma = sqrt(0.5 * np);
   for (int r0 = (g.frame - 1) / kF64Round * kF64Round; r0 >= 0; r0 -= kF64Round) {
     const int blocks = (min(kF64Round, g.frame - r0) + kF64Block - 1) / kF64Block;
-    const int n0 = r0 + kF64Run * tid;
+    const int n0 = r0 + RUN * tid;
     const bool active = n0 < g.frame;
-    double2 z[kF64Run];
+    double2 z[RUN];
 #pragma unroll
-    for (int b = 0; b < kF64Run; ++b) z[b] = make_double2(0.0, 0.0);
+    for (int b = 0; b < RUN; ++b) z[b] = make_double2(0.0, 0.0);
     for (int p = 0; p < L; ++p) {
       if (!path_in_range(a, p)) continue;
       const int d = a.delays[p];
-      double2 h[kF64Run];
+      double2 h[RUN];
 #pragma unroll
-      for (int b = 0; b < kF64Run; ++b) h[b] = make_double2(0.0, 0.0);
+      for (int b = 0; b < RUN; ++b) h[b] = make_double2(0.0, 0.0);
       for (int t0 = 0; t0 < terms; t0 += g.term_group) {
         const int tg = min(g.term_group, terms - t0);
         // tables [tg][blocks | 8 | 8]
@@ -818,17 +824,17 @@ f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
         if (active) {
           const double2* tq = y + (n0 - r0) / kF64Block;
           const double2* ta = y + blocks + ((n0 / kF64Run) & (kF64Block / kF64Run - 1));
-          const double2* tb = y + blocks + kF64Run;
+          const double2* tb = y + blocks + kF64Run + (n0 & (kF64Run - 1));
           for (int k = 0; k < tg; ++k) {
             const double2 c = dcmul(tq[k * row], ta[k * row]);
 #pragma unroll
-            for (int b = 0; b < kF64Run; ++b) h[b] = dcfma(c, tb[k * row + b], h[b]);
+            for (int b = 0; b < RUN; ++b) h[b] = dcfma(c, tb[k * row + b], h[b]);
           }
         }
       }
       if (active) {
 #pragma unroll
-        for (int b = 0; b < kF64Run; ++b) {
+        for (int b = 0; b < RUN; ++b) {
           const int m = n0 + b - d;  // (x holds dx >= d zeros before the frame)
           if (n0 + b < g.frame) z[b] = dcfma(h[b], x[g.dx + m], z[b]);
         }
@@ -837,12 +843,12 @@ f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
     __syncthreads();
     if (active) {
 #pragma unroll
-      for (int b = 0; b < kF64Run; b += 2) {
+      for (int b = 0; b < RUN; b += 2) {
         // noise sample i: words (0, 1) of call i / 2 for even i, (2, 3) for odd i
         const uint4 wn = stream_call(a.seed, drop, HPX_STREAM_NOISE, static_cast<uint32_t>((n0 + b) >> 1));
 #pragma unroll
-        for (int o = 0; o < 2; ++o) {
-          const int i = n0 + b + o;
+        for (int j = 0; j < (RUN > 1 ? 2 : 1); ++j) {
+          const int i = n0 + b + j, o = RUN > 1 ? j : i & 1;
           if (i >= g.frame) break;
           const uint32_t w0 = o ? wn.z : wn.x, w1 = o ? wn.w : wn.y;
           const double u1 = (static_cast<double>(w0 >> 8) + 0.5) * 5.9604644775390625e-08;
@@ -850,7 +856,7 @@ f64_drop_kernel(BatchArgs a, F64Layout g, double2* equalized) {
           const double rho = sigma * sqrt(-2.0 * log(u1));
           double ns, nc;
           sincospi(2.0 * u2, &ns, &nc);
-          const double2 v = dcmul(S, z[b + o]);
+          const double2 v = dcmul(S, z[b + j]);
           y[i] = make_double2(fma(rho, nc, v.x), fma(rho, ns, v.y));
         }
       }
@@ -923,36 +929,45 @@ extern "C" int hpx_run_batch_f64(const hpx_link* link_host, const int32_t* delay
   g.dx = a.maxd;
   g.frame = a.words * (a.n + a.cp);
   g.bits_words = static_cast<int>((static_cast<int64_t>(a.words) * a.n * a.bps + 31) / 32) + 1;
-  int64_t o = 0;
-  auto take = [&](int64_t bytes) {
-    const int at = static_cast<int>(o);
-    o += align16(bytes);
-    return at;
-  };
-  // the prologue's uniforms alias the transmit buffer where it is long enough, which it is for every
-  // frame but the shortest; the sinusoids' tables alias the receive buffer
-  const int64_t uni_elems = (static_cast<int64_t>(a.nnorm) + 1) / 2;  // in complex128 values
-  g.off_sos = take(static_cast<int64_t>(a.paths) * a.terms * 3 * sizeof(double));
-  g.off_tw = take(static_cast<int64_t>(a.n) * sizeof(double2));
-  g.off_x = take(std::max<int64_t>(g.dx + g.frame, uni_elems) * sizeof(double2));
-  g.off_y = take(static_cast<int64_t>(g.frame) * sizeof(double2));
-  g.off_abar = take(static_cast<int64_t>(a.paths) * a.words * sizeof(double2));
-  g.off_bits = take(static_cast<int64_t>(g.bits_words) * sizeof(uint32_t));
-  g.off_red = take(16);
-  // (a frame has at least 32 samples: one term's table always fits)
+  // a round's rows of the tables; a frame too short for the tables of all sinusoids gets room for them (in groups
+  // they cost two barriers each: 32 subcarriers, one word, 15 paths 177 us in groups of two, 119 at once)
   const int round = std::min(g.frame, kF64Round);
-  g.term_group = std::max(1, round / ((round + kF64Block - 1) / kF64Block + 2 * kF64Run));
-  g.bytes = o;
+  const int row = (round + kF64Block - 1) / kF64Block + 2 * kF64Run;
+  auto layout = [&](int work) {
+    int64_t o = 0;
+    auto take = [&](int64_t bytes) {
+      const int at = static_cast<int>(o);
+      o += align16(bytes);
+      return at;
+    };
+    // the prologue's uniforms alias the transmit buffer where it is long enough, which it is for every
+    // frame but the shortest; the sinusoids' tables alias the receive buffer
+    const int64_t uni_elems = (static_cast<int64_t>(a.nnorm) + 1) / 2;  // in complex128 values
+    g.work = work;
+    g.off_sos = take(static_cast<int64_t>(a.paths) * a.terms * 3 * sizeof(double));
+    g.off_tw = take(static_cast<int64_t>(a.n) * sizeof(double2));
+    g.off_x = take(std::max<int64_t>(g.dx + g.frame, uni_elems) * sizeof(double2));
+    g.off_y = take(static_cast<int64_t>(work) * sizeof(double2));
+    g.off_abar = take(static_cast<int64_t>(a.paths) * a.words * sizeof(double2));
+    g.off_bits = take(static_cast<int64_t>(g.bits_words) * sizeof(uint32_t));
+    g.off_red = take(16);
+    // (a frame has at least 32 samples: one term's table always fits)
+    g.term_group = std::max(1, std::max(round, std::min(work, kF64Round)) / row);
+    g.bytes = o;
+  };
+  layout(std::max(g.frame, std::min(a.terms * row, kF64Tables)));
+  if (g.bytes > kMaxLds) layout(g.frame);
   if (g.bytes > kMaxLds) {
     set_error("hpx_run_batch_f64: %lld bytes of LDS per drop exceed a CU's %lld", static_cast<long long>(g.bytes),
               static_cast<long long>(kMaxLds));
     return HPX_ERR_UNSUPPORTED;
   }
-  if (!ensure_lds(reinterpret_cast<const void*>(f64_drop_kernel), g.bytes)) {
+  const auto kernel = g.frame <= kF64Threads ? f64_drop_kernel<1> : f64_drop_kernel<kF64Run>;
+  if (!ensure_lds(reinterpret_cast<const void*>(kernel), g.bytes)) {
     set_error("hpx_run_batch_f64: %lld bytes of LDS per workgroup not available", static_cast<long long>(g.bytes));
     return HPX_ERR_UNSUPPORTED;
   }
-  hipLaunchKernelGGL(f64_drop_kernel, dim3(static_cast<unsigned>(num_drops)), dim3(kF64Threads),
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(num_drops)), dim3(kF64Threads),
                      static_cast<size_t>(g.bytes), static_cast<hipStream_t>(stream), a,
                      g, reinterpret_cast<double2*>(equalized));
   return check_launch("hpx_run_batch_f64");

@@ -171,6 +171,7 @@ int make_plan(const hpx_link* l, const hpx_frame* f, Plan* out, bool allow_lean 
   }
   out->threads = threads;
   out->pairs = pairs;
+  out->antennas = nt;
   {
     const int maxt = threads <= 256 ? 256 : 512;
     const int def = fft_values_for(nt, maxt), alt = alt_fft_values_for(nt, maxt);
@@ -516,22 +517,32 @@ extern "C" int hpx_run_batch_drops(const hpx_link* link_host, const hpx_frame* f
     return HPX_ERR_UNSUPPORTED;
   }
   if (num_drops == 0) return HPX_OK;
-  const bool eight = link_host->num_tx == 8;
-  if (link_host->workgroup_size == 0 && link_host->num_subcarriers <= (eight ? 128 : 64)) {
-    // A launch that fills the GPU: one-wavefront workgroups do without the larger one's idle wavefronts and
-    // barriers where the LDS lets a CU hold 16 of them or, with 8 antennas, more wavefronts (at most 8, by
-    // registers) than with words side by side.  64 subcarriers, 5 paths: 4096 drops 145 instead of 173 us,
-    // 8192 drops 264 instead of 331 us (2048: 105 instead of 91); 8x8 with 128 subcarriers, 6 paths: 4000
-    // drops 1146 instead of 1258 us.
-    hpx_link narrow = *link_host;
-    narrow.workgroup_size = 64;
-    Plan np;
-    if (make_plan(&narrow, frame_host, &np) == HPX_OK && plan.launch_threads > 64) {
-      const int64_t most = eight ? 8 : 16;
-      const int64_t wide = std::min(most, kMaxLds / plan.lds * (plan.launch_threads / 64));
-      const int64_t fill = resident_workgroups(most, 64, np.lds);
-      if (kMaxLds / np.lds > (eight ? wide : most - 1) && num_drops >= (eight ? fill - fill / 8 : fill))
-        plan = np;
+  if (link_host->workgroup_size == 0 && link_host->num_subcarriers <= 2 * kBatchThreads) {
+    // Workgroups of 64 to batch_threads() threads, words side by side where that leaves threads idle: large ones take
+    // fewer steps over a drop's words, small ones leave the GPU room for more drops, whose prologues hardly
+    // gain from threads.  The shorter launch by the model of segments_for; of drops that fill the GPU the
+    // one-word workgroup (N / 2 threads) unless another wins clearly.  1x1, 6 paths, 64, 128 and 256 threads: 128 subcarriers and one word, 20000
+    // drops 255, 366 and 597 us, 2000 drops 43, 43 and 70; 14 words, 20000 drops 1450, 1242 and 1426 us, 700 drops
+    // 96, 89 and 79; 256 subcarriers and 3 words, 20000 drops 506, 612 and 834 us.
+    const int cus = device_cus(), waves = link_host->num_tx == 8 ? 8 : 16;
+    const int one_word = std::max(64, link_host->num_subcarriers / 2);
+    const bool full = num_drops > cus * workgroups_per_cu(waves, plan.launch_threads, plan.lds);
+    auto time_of = [&](const Plan& p) {
+      return plan_segments(p, num_drops, waves, cus).time * (full && p.launch_threads == one_word ? 0.9 : 1.0);
+    };
+    double best = time_of(plan);
+    const int made = plan.launch_threads;
+    for (int t = 64; t <= batch_threads(link_host->num_tx); t *= 2) {
+      if (t == made || link_host->num_subcarriers > 4 * t) continue;
+      hpx_link other = *link_host;
+      other.workgroup_size = t;
+      Plan p;
+      if (make_plan(&other, frame_host, &p) != HPX_OK) continue;
+      const double time = time_of(p);
+      if (time < best) {
+        best = time;
+        plan = p;
+      }
     }
   }
   BatchArgs& a = plan.args;

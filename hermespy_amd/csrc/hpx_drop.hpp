@@ -773,33 +773,61 @@ inline int waves_per_cu(const void* fn) {
   return 4 * std::min(8, 512 / ((attr.numRegs + 7) & ~7));
 }
 
-// Workgroups the GPU holds at once, by LDS and by registers.
-inline int64_t resident_workgroups(int cu_waves, int threads, int64_t lds) {
+inline int device_cus() {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
+  return cus;
+}
+
+// Workgroups a CU holds at once, by LDS and by registers.
+inline int64_t workgroups_per_cu(int cu_waves, int threads, int64_t lds) {
   const int64_t by_waves = static_cast<int64_t>(cu_waves) * 64 / threads;
-  return cus * std::max<int64_t>(1, std::min<int64_t>(kMaxLds / std::max<int64_t>(lds, 1), by_waves));
+  return std::max<int64_t>(1, std::min<int64_t>(kMaxLds / std::max<int64_t>(lds, 1), by_waves));
 }
 
 // Workgroups a drop's words are spread over.  The drops of a small launch leave much of the GPU idle
 // while each steps through its words, and a launch of a little more than the GPU holds leaves it
-// idle in its second round, so a drop is cut into the segments for which rounds x length is shortest:
-// a segment repeats the prologue (some kPrologue of a drop's time), and the word before it where
-// delays reach into it.  One drop of 64 subcarriers 131 -> 31 us, one 4x4 drop of 1024 subcarriers 355 ->
-// 63 us, 1000 2x2 drops of 512 subcarriers with exports 586 -> 441 us.
-constexpr double kPrologue = 0.15;
-template <class Resident>
-int segments_for(int64_t drops, int most, Resident resident) {
-  int best = 1;
-  double cost = 0.0;
+// idle in its second round, so a drop is cut into the segments for which a launch is shortest: rounds of
+// the GPU times what a segment takes, its prologue and its steps.  A segment repeats the prologue, whatever the
+// frame's length, and a part of the word before it where delays reach into it, and a launch that zeroes the
+// errors goes before.  A full GPU slows prologue and steps, so the last round costs less the emptier it is.
+// Times in word steps, of 10 us (1x1 at 64 subcarriers) to 35 us (8x8 at 1024), from launches of 1 to 20000 drops of 1 to
+// 40 words: of 916 such shapes of 32 to 1024 subcarriers and 1 to 8 antennas the choice is slower than whole drops of
+// N / 2 threads in MODEL_FIG.  One drop of 64 subcarriers 131 -> 31 us, one 4x4 drop of
+// 1024 subcarriers 355 -> 63 us, 1000 2x2 drops of 512 subcarriers with exports 586 -> 441 us; 700 4x4 drops of 1024
+// subcarriers and 3 words stay whole, 165 us, 216 in two segments.
+constexpr double kLead = 0.35, kZero = 0.3;
+constexpr double kStepFull = 0.36;  // what a full GPU adds to a step
+
+// A workgroup's prologue, what a full GPU adds to it, and a step of its threads.
+struct GroupTimes {
+  double prologue, prologue_full, step;
+};
+inline GroupTimes group_times(int nt, int threads, bool batch) {
+  const double one = nt == 1 ? 2.3 : nt == 2 ? 2.0 : 1.6;  // (the detector of more antennas hides behind the rest)
+  // one wavefront does the detector after the rest, and waits for each step alone
+  if (threads <= 64) return {one + (nt == 1 ? 0.2 : nt == 2 ? 0.4 : 0.6), 0.5, nt == 8 ? 1.0 : batch ? 1.25 : 1.1};
+  return threads <= 128 ? GroupTimes{one + 0.1, 0.36, 1.0} : GroupTimes{one, 0.28, threads <= 256 ? 0.9 : 1.0};
+}
+// Time of a launch of `groups` workgroups of `steps` steps of which the GPU holds `resident`.
+inline double launch_time(const GroupTimes& g, int64_t groups, int64_t resident, double steps) {
+  const int64_t rounds = groups / resident;
+  const double rest = static_cast<double>(groups - rounds * resident) / static_cast<double>(resident);
+  auto in_rounds = [&](double full) { return static_cast<double>(rounds) * (1.0 + full) + (rest > 0.0 ? 1.0 + full * rest : 0.0); };
+  return g.prologue * in_rounds(g.prologue_full) + steps * g.step * in_rounds(kStepFull);
+}
+struct Segments {
+  int count = 1;
+  double time = 0.0;  // of the launch
+};
+// steps(s): steps of the longest of s segments; resident(s): segments the GPU holds
+template <class Steps, class Resident>
+Segments segments_for(const GroupTimes& g, int64_t drops, int most, double lead, Steps steps, Resident resident) {
+  Segments best;
   for (int s = 1; s <= most; ++s) {
-    const int64_t r = resident(s);
-    const double c = static_cast<double>((drops * s + r - 1) / r) * (kPrologue + (1.0 - kPrologue) / s);
-    if (s == 1 || c < cost) {
-      best = s;
-      cost = c;
-    }
+    const double t = launch_time(g, drops * s, resident(s), steps(s) + (s > 1 ? lead : 0.0)) + (s > 1 ? kZero : 0.0);
+    if (s == 1 || t < best.time) best = {s, t};
   }
   return best;
 }
@@ -808,6 +836,7 @@ int segments_for(int64_t drops, int most, Resident resident) {
 // 1000 and 2048 drops 1763, 3207, 2373 and 3076 us with lean drops whole, 844, 1272, 1620 and 2904 us in up to
 // four segments, 652, 897, 1631 and 2963 us in up to seven.
 constexpr int kMultiMaxSegments = 7;
+constexpr double kMultiWords = 14.0;
 
 // Raises a kernel's dynamic LDS limit once per process and size (so that launches recorded
 // into a graph after a first eager run make no attribute calls).
@@ -843,8 +872,9 @@ int launch_multi_kernel(const BatchArgs* plans, const hpx_uneven_class& c, hipSt
   const BatchArgs* first = plans + c.first;
   const int threads = batched_class(NT, c.threads, c.pairs) ? batch_threads(NT) : c.threads;
   const int64_t resident =
-      resident_workgroups(waves_per_cu(reinterpret_cast<const void*>(fn)), threads, c.lds_bytes);
-  const int segs = segments_for(c.count, kMultiMaxSegments, [&](int) { return resident; });
+      device_cus() * workgroups_per_cu(waves_per_cu(reinterpret_cast<const void*>(fn)), threads, c.lds_bytes);
+  const int segs = segments_for(group_times(NT, threads, threads > c.threads), c.count, kMultiMaxSegments, 0.0,
+                                [](int s) { return kMultiWords / s; }, [&](int) { return resident; }).count;
   if (LEAN && segs > 1)  // the workspaces first
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(c.count)), dim3(threads), c.lds_bytes, stream, first, 0);
   else if (segs > 1)
@@ -871,6 +901,7 @@ int launch_multi_fftv(const BatchArgs* plans, const hpx_uneven_class& c, hipStre
 struct Plan {
   int threads = 0, pairs = 0;  // threads per word, sample pairs per thread
   int launch_threads = 0;      // workgroup size
+  int antennas = 0;
   int segs = 1;                // segments per drop (single-link launches)
   bool batch = false;          // several words side by side
   int fftv = 0;  // FFT values per thread and pass
@@ -880,25 +911,38 @@ struct Plan {
   BatchArgs args{};
 };
 
-// Cuts the drops of a single-link launch into segments: a segment's Taylor table holds the blocks of its
-// own words only, which shortens the LDS layout after it.
-inline void set_segments(Plan* plan, int64_t num_drops, int cu_waves) {
-  BatchArgs& a = plan->args;
+// Blocks of a segment's Taylor table, of its own words only, and the bytes of a table.
+inline int segment_blocks(const BatchArgs& a, int segs) {
+  if (segs == 1) return a.nb;
   const int64_t period = a.n + a.cp;
-  auto blocks = [&](int segs) {  // most blocks a segment's windows and delays touch
-    if (segs == 1) return a.nb;
-    const int64_t span = (a.words + segs - 1) / segs * period + std::max(0, a.maxd - a.cp);
-    return static_cast<int>(std::min<int64_t>(a.nb, ((span - 2) >> a.log2b) + 2));
-  };
-  auto table = [&](int nb) { return align16(static_cast<int64_t>(a.paths) * nb * kTaylorCoeffs * sizeof(float2)); };
-  const int full = a.nb;
-  const int segs = segments_for(num_drops, (a.words + a.wb - 1) / a.wb, [&](int s) {
-    return resident_workgroups(cu_waves, plan->launch_threads, plan->lds - table(full) + table(blocks(s)));
-  });
+  const int64_t span = (a.words + segs - 1) / segs * period + std::max(0, a.maxd - a.cp);
+  return static_cast<int>(std::min<int64_t>(a.nb, ((span - 2) >> a.log2b) + 2));
+}
+inline int64_t table_bytes(const BatchArgs& a, int nb) {
+  return align16(static_cast<int64_t>(a.paths) * nb * kTaylorCoeffs * sizeof(float2));
+}
+
+// Segments of a single-link launch on `cus` CUs whose registers allow cu_waves wavefronts each.
+inline Segments plan_segments(const Plan& plan, int64_t num_drops, int cu_waves, int cus) {
+  const BatchArgs& a = plan.args;
+  // a thread's second sample pair nearly doubles a step (1x1 at 256 subcarriers on 64 threads)
+  const double step = a.n > 2 * plan.launch_threads ? 0.95 * a.n / (2 * plan.launch_threads) : 1.0;
+  return segments_for(
+      group_times(plan.antennas, plan.launch_threads, plan.batch), num_drops, (a.words + a.wb - 1) / a.wb, a.dx > 0 ? kLead : 0.0,
+      [&](int s) { return step * (((a.words + s - 1) / s + a.wb - 1) / a.wb); },
+      [&](int s) {
+        const int64_t lds = plan.lds - table_bytes(a, a.nb) + table_bytes(a, segment_blocks(a, s));
+        return cus * workgroups_per_cu(cu_waves, plan.launch_threads, lds);
+      });
+}
+
+// Cuts the drops of a single-link launch: the shorter Taylor table shortens the LDS layout after it.
+inline void set_segments(Plan* plan, int segs) {
   if (segs == 1) return;
+  BatchArgs& a = plan->args;
   plan->segs = segs;
-  const int nb = blocks(segs);
-  const int less = static_cast<int>(table(full) - table(nb));
+  const int nb = segment_blocks(a, segs);
+  const int less = static_cast<int>(table_bytes(a, a.nb) - table_bytes(a, nb));
   a.nb = nb;
   plan->lds -= less;
   for (int* off : {&a.off_abar, &a.off_tw, &a.off_bits, &a.off_cons, &a.off_s, &a.off_det, &a.off_red, &a.off_dly, &a.off_dmb,
@@ -908,7 +952,7 @@ inline void set_segments(Plan* plan, int64_t num_drops, int cu_waves) {
 
 template <class K>
 int launch(K kernel, Plan plan, int64_t num_drops, hipStream_t stream) {
-  set_segments(&plan, num_drops, waves_per_cu(reinterpret_cast<const void*>(kernel)));
+  set_segments(&plan, plan_segments(plan, num_drops, waves_per_cu(reinterpret_cast<const void*>(kernel)), device_cus()).count);
   if (!ensure_lds(reinterpret_cast<const void*>(kernel), plan.lds)) {
     set_error("hpx_run_batch: %lld bytes of LDS per workgroup not available", static_cast<long long>(plan.lds));
     return HPX_ERR_UNSUPPORTED;

@@ -739,7 +739,15 @@ __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(batch
 batch_kernel_multi(const BatchArgs* __restrict__ plans, int segs) {
   const int parts = LEAN && segs == 0 ? 1 : segs;
   const int slot = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / parts);
-  drop_body<NT, NR, PAIRS, FFTV, LEAN, true, BATCH>((ConstArgs*)(plans + slot), 0, static_cast<int>(blockIdx.x) - slot * parts, segs);
+  const int seg = static_cast<int>(blockIdx.x) - slot * parts;
+  // a drop of fewer steps than the launch has segments makes one segment a step; the others would only repeat its prologue
+  ConstArgs* plan = (ConstArgs*)(plans + slot);
+  if (segs > 1) {
+    const int most = (plan->words + plan->wb - 1) / plan->wb;
+    if (seg >= most) return;
+    segs = min(segs, most);
+  }
+  drop_body<NT, NR, PAIRS, FFTV, LEAN, true, BATCH>(plan, 0, seg, segs);
 }
 
 // Zero error counts of drops whose segments add to them (a kernel, so that a captured graph holds no
@@ -794,7 +802,7 @@ inline int64_t workgroups_per_cu(int cu_waves, int threads, int64_t lds) {
 // errors goes before.  A full GPU slows prologue and steps, so the last round costs less the emptier it is.
 // Times in word steps, of 10 us (1x1 at 64 subcarriers) to 35 us (8x8 at 1024), from launches of 1 to 20000 drops of 1 to
 // 40 words: of 916 such shapes of 32 to 1024 subcarriers and 1 to 8 antennas the choice is slower than whole drops of
-// N / 2 threads in MODEL_FIG.  One drop of 64 subcarriers 131 -> 31 us, one 4x4 drop of
+// N / 2 threads by at most 5 %, and 1.65 times as fast in the mean.  One drop of 64 subcarriers 131 -> 31 us, one 4x4 drop of
 // 1024 subcarriers 355 -> 63 us, 1000 2x2 drops of 512 subcarriers with exports 586 -> 441 us; 700 4x4 drops of 1024
 // subcarriers and 3 words stay whole, 165 us, 216 in two segments.
 constexpr double kLead = 0.35, kZero = 0.3;
@@ -831,12 +839,14 @@ Segments segments_for(const GroupTimes& g, int64_t drops, int most, double lead,
   }
   return best;
 }
-// (A class's words per drop are known to its plans only.)  Lean drops, one of which a CU holds and which take
-// 1.5 ms each in one piece, are cut too, after a launch that fills their workspaces: mixed batches of 64, 300,
-// 1000 and 2048 drops 1763, 3207, 2373 and 3076 us with lean drops whole, 844, 1272, 1620 and 2904 us in up to
-// four segments, 652, 897, 1631 and 2963 us in up to seven.
+// Heterogeneous classes: their words per drop are known to the plans only (a drop makes no more segments than it has
+// steps), and they share the GPU with the classes of other streams, so a class's segments fill at most half of it.  Lean
+// drops, one of which a CU holds and which take 1.5 ms each in one piece, are cut too, after a launch that fills
+// their workspaces.  Mixed batches of 64, 300, 1000, 2048 and 8192 drops on four streams: whole 2754, 3970, 3591, 3678 and
+// 8211 us, in segments that may fill the GPU 660, 897, 1600, 2893 and 8587, half of it 671, 894, 1584, 2736 and
+// 8247; of 3 words each instead of 14, 2048 and 8192 drops 1021 and 2172, 1260 and 2448, 922 and 2156.
 constexpr int kMultiMaxSegments = 7;
-constexpr double kMultiWords = 14.0;
+constexpr double kMultiWords = 14.0;  // a drop's steps, for the rule's sake
 
 // Raises a kernel's dynamic LDS limit once per process and size (so that launches recorded
 // into a graph after a first eager run make no attribute calls).
@@ -873,7 +883,8 @@ int launch_multi_kernel(const BatchArgs* plans, const hpx_uneven_class& c, hipSt
   const int threads = batched_class(NT, c.threads, c.pairs) ? batch_threads(NT) : c.threads;
   const int64_t resident =
       device_cus() * workgroups_per_cu(waves_per_cu(reinterpret_cast<const void*>(fn)), threads, c.lds_bytes);
-  const int segs = segments_for(group_times(NT, threads, threads > c.threads), c.count, kMultiMaxSegments, 0.0,
+  const int most = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kMultiMaxSegments, resident / (2 * c.count))));
+  const int segs = segments_for(group_times(NT, threads, threads > c.threads), c.count, most, 0.0,
                                 [](int s) { return kMultiWords / s; }, [&](int) { return resident; }).count;
   if (LEAN && segs > 1)  // the workspaces first
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(c.count)), dim3(threads), c.lds_bytes, stream, first, 0);

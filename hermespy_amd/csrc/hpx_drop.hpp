@@ -725,11 +725,11 @@ constexpr int batch_waves_per_eu() {
 
 template <int NT, int NR, int PAIRS, int MAXT, bool BATCH = false>
 __global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(batch_waves_per_eu<NT, PAIRS, MAXT>())))
-batch_kernel(BatchArgs a, int segs) {
+batch_kernel(BatchArgs a, int segs, int first) {
   const int drop = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) / segs);
   // (the arguments where they lie: a is the kernel's first parameter)
   drop_body<NT, NR, PAIRS, fft_values<NT, MAXT>(), false, compact_uniforms(MAXT), BATCH>(
-      (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr(), drop, static_cast<int>(blockIdx.x) - drop * segs, segs);
+      (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr(), first + drop, static_cast<int>(blockIdx.x) - drop * segs, segs);
 }
 
 // Heterogeneous batches: workgroup i simulates the drop plans[i] describes; its first_drop is
@@ -780,6 +780,9 @@ inline int waves_per_cu(const void* fn) {
   if (hipFuncGetAttributes(&attr, fn) != hipSuccess || attr.numRegs <= 0) return 8;
   return 4 * std::min(8, 512 / ((attr.numRegs + 7) & ~7));
 }
+
+// Drops of `threads` threads each in one launch, which holds fewer than 2^32.
+inline int64_t drops_per_launch(int threads) { return 0xffffffffll / threads; }
 
 inline int device_cus() {
   int dev = 0, cus = 256;
@@ -879,19 +882,24 @@ int launch_multi_kernel(const BatchArgs* plans, const hpx_uneven_class& c, hipSt
     set_error("hpx_uneven_run: %lld bytes of LDS per workgroup not available", static_cast<long long>(c.lds_bytes));
     return HPX_ERR_UNSUPPORTED;
   }
-  const BatchArgs* first = plans + c.first;
+  const BatchArgs* const all = plans + c.first;
   const int threads = batched_class(NT, c.threads, c.pairs) ? batch_threads(NT) : c.threads;
   const int64_t resident =
       device_cus() * workgroups_per_cu(waves_per_cu(reinterpret_cast<const void*>(fn)), threads, c.lds_bytes);
   const int most = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kMultiMaxSegments, resident / (2 * c.count))));
   const int segs = segments_for(group_times(NT, threads, threads > c.threads), c.count, most, 0.0,
                                 [](int s) { return kMultiWords / s; }, [&](int) { return resident; }).count;
-  if (LEAN && segs > 1)  // the workspaces first
-    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(c.count)), dim3(threads), c.lds_bytes, stream, first, 0);
-  else if (segs > 1)
-    hipLaunchKernelGGL(zero_plan_errors_kernel, dim3(static_cast<unsigned>((c.count + 255) / 256)), dim3(256), 0, stream,
-                       first, static_cast<int>(c.count));
-  hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(c.count * segs)), dim3(threads), c.lds_bytes, stream, first, segs);
+  const int64_t pieces = drops_per_launch(threads * segs);
+  for (int64_t at = 0; at < c.count; at += pieces) {
+    const BatchArgs* const first = all + at;
+    const int64_t count = std::min(pieces, c.count - at);
+    if (LEAN && segs > 1)  // the workspaces first
+      hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(count)), dim3(threads), c.lds_bytes, stream, first, 0);
+    else if (segs > 1)
+      hipLaunchKernelGGL(zero_plan_errors_kernel, dim3(static_cast<unsigned>((count + 255) / 256)), dim3(256), 0, stream,
+                         first, static_cast<int>(count));
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(count * segs)), dim3(threads), c.lds_bytes, stream, first, segs);
+  }
   return check_launch("hpx_uneven_run");
 }
 
@@ -971,8 +979,10 @@ int launch(K kernel, Plan plan, int64_t num_drops, hipStream_t stream) {
   if (plan.segs > 1)
     hipLaunchKernelGGL(zero_errors_kernel, dim3(static_cast<unsigned>((num_drops + 255) / 256)), dim3(256), 0, stream,
                        plan.args.errors, static_cast<int>(num_drops));
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(num_drops * plan.segs)), dim3(plan.launch_threads), plan.lds,
-                     stream, plan.args, plan.segs);
+  const int64_t most = drops_per_launch(plan.launch_threads * plan.segs);
+  for (int64_t first = 0; first < num_drops; first += most)
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(std::min(most, num_drops - first) * plan.segs)),
+                       dim3(plan.launch_threads), plan.lds, stream, plan.args, plan.segs, static_cast<int>(first));
   return check_launch("hpx_run_batch");
 }
 

@@ -48,3 +48,24 @@ def test_lmmse_rows(cuda):
             x, got = ls[t, part:part + rows // 8], est[t, part:part + rows // 8]
             error = torch.view_as_real(got - x * filt[t, 0, 0]).abs().amax(dim=-1)
             assert bool((error <= 4 * 2.0**-24 * 2 * x.abs() * filt[t, 0, 0].abs()).all())
+
+
+# 256 threads a drop, and the library's choice for a launch that fills the GPU many times over
+@pytest.mark.parametrize("workgroup,drops", [(256, (1 << 24) + 1000), (0, (1 << 25) + 1000)])
+def test_drops(cuda, workgroup, drops):
+    """The drops at both ends of a launch of 2^32 threads and more are those of launches of their own."""
+
+    import dataclasses
+
+    from hermespy_amd.configs import siso_64
+    from hermespy_amd.simulation import BatchedLink
+
+    link = BatchedLink(dataclasses.replace(siso_64(), workgroup_size=workgroup))
+    noise = torch.full((drops,), 0.1, dtype=torch.float64, device=cuda)
+    errors = torch.full((drops,), -1, dtype=torch.int32, device=cuda)
+    link.run(11, 0, noise, errors)
+    assert int(errors.min()) >= 0
+    for first in (0, (1 << 24) - 500, drops - 1000):
+        alone = torch.full((1000,), -1, dtype=torch.int32, device=cuda)
+        link.run(11, first, noise[:1000].contiguous(), alone)
+        assert torch.equal(alone, errors[first:first + 1000])

@@ -904,10 +904,10 @@ net_forward_kernel(const float2* __restrict__ grid, int num_drops, int num_rx, i
       }
     });
     sample_sync<PT>();
-    // the activations from LDS, in whole lines (eight bytes a lane from the accumulators touch 32 lines a store: a
-    // training forward pass of 4096 samples 332 us, 287 now)
+    // the activations from LDS, in whole lines (eight bytes a lane from the accumulators touch 32 lines a store)
     if constexpr (TRAIN) {
-      constexpr int kLanes = PT == 1 ? 128 : 64;
+      constexpr int kLanes = 128;  // a sample's two wavefronts
+      static_assert(PT == 1, "");
       const int g = ln.template sample<PT>(0);
       if (s0 + g < num_samples) {
         uint16_t* dst = kept.act[layer] + (s0 + g) * kActElems;
@@ -1080,10 +1080,19 @@ net_backward_kernel(const uint16_t* __restrict__ dz_out, int64_t num_samples, Gr
   gradient(0);
 }
 
-// Tiles per wavefront: two (four samples a workgroup) where that still leaves two workgroups for each of the
-// 256 CUs, else one: 2044 samples 80 us with one, 2080 samples 91 us with two (88 and 145 us before), one drop
-// of four samples 38 us (58).
-int fused_tiles(int64_t samples) { return samples >= 4 * 512 ? 2 : 1; }
+// Tiles per wavefront of the estimator: one (two samples a workgroup, four workgroups a CU, so eight samples a
+// CU at a time) or two (four samples, three workgroups, twelve), whichever takes the shorter rounds: a full round of
+// one takes 0.79 of the time of two.  224 output channels, one and two: 2048 samples 77 and 78 us, 2052 109 and 91,
+// 3072 121 and 99, 3300 131 and 147, 4096 152 and 158, 5000 195 and 180, 16384 592 and 534.  The training forward pass,
+// which stores what the backward pass needs, takes one tile at every size: 2052 samples 128 and 123 us, 3072 159 and 235,
+// 4096 214 and 321, 16384 788 and 1199.
+int fused_tiles(int64_t samples) {
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) == hipSuccess)
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
+  const auto rounds = [&](int64_t a_round) { return static_cast<double>((samples + a_round - 1) / a_round); };
+  return 0.79 * rounds(8 * cus) <= rounds(12 * cus) ? 1 : 2;
+}
 
 unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
@@ -1287,16 +1296,10 @@ extern "C" int hpx_net_forward(const uint16_t* x, int64_t num_samples, const uin
     all |= reinterpret_cast<uintptr_t>(pre[i]) | reinterpret_cast<uintptr_t>(act[i]);
   }
   HPX_REQUIRE((all & 15u) == 0, "hpx_net_forward: arrays must be 16-byte aligned");
-  const int pt = fused_tiles(num_samples);
-  const dim3 g(static_cast<unsigned>((num_samples + 2 * pt - 1) / (2 * pt)));
-#define HPX_FORWARD(PT)                                                                                                  \
-  hipLaunchKernelGGL((net_forward_kernel<PT, true, true>), g, dim3(256), 0, as_stream(stream),                          \
-                     static_cast<const float2*>(nullptr), 0, 0, 0, 0, static_cast<const int32_t*>(nullptr),             \
-                     static_cast<const float2*>(nullptr), 0, static_cast<const double*>(nullptr), x, num_samples, net,  \
-                     cout, static_cast<float*>(nullptr), kept)
-  if (pt == 2) HPX_FORWARD(2);
-  else HPX_FORWARD(1);
-#undef HPX_FORWARD
+  hipLaunchKernelGGL((net_forward_kernel<1, true, true>), dim3(static_cast<unsigned>((num_samples + 1) / 2)), dim3(256), 0,
+                     as_stream(stream), static_cast<const float2*>(nullptr), 0, 0, 0, 0, static_cast<const int32_t*>(nullptr),
+                     static_cast<const float2*>(nullptr), 0, static_cast<const double*>(nullptr), x, num_samples, net, cout,
+                     static_cast<float*>(nullptr), kept);
   return check_launch("hpx_net_forward");
 }
 

@@ -110,7 +110,7 @@ int make_plan(const hpx_link* l, const hpx_frame* f, Plan* out, bool allow_lean 
   a.bps = mod.bps;
   a.order = l->modulation_order;
   a.mod = mod;
-  a.dbounds = demap_bounds(mod);
+  a.dbounds = demap_bounds_of(mod);
   a.detector = l->detector;
   a.dc = l->dc_suppression ? 1 : 0;
   a.paths = l->num_paths;

@@ -10,7 +10,6 @@
 #include <math.h>
 
 #include <algorithm>
-#include <array>
 
 #include "hpx_common.hpp"
 #include "hpx_detect.hpp"
@@ -309,19 +308,6 @@ int detect_segments(int64_t drops, int64_t drop_bytes, int words, int64_t elemen
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(most, target / std::max<int64_t>(drops, 1))));
 }
 
-// The boundaries of the four constellations, found once (500 steps of a bisection: a tenth of a small call).
-const DemapBounds& bounds_of(const Modulation& mod) {
-  static const auto all = [] {
-    std::array<DemapBounds, 4> b{};
-    for (int i = 0; i < 4; ++i) {
-      Modulation m;
-      if (modulation(4 << (2 * i), 1, &m)) b[i] = demap_bounds(m);
-    }
-    return b;
-  }();
-  return all[mod.bps / 2 - 1];
-}
-
 template <int NT>
 int detect_launch(const Modulation& mod, const float2* grid, const float2* est, int num_drops, int num_rx, int words, int n,
                   const int32_t* elements, const int32_t* word_data, int mmse, const double* noise_power, uint64_t seed,
@@ -332,7 +318,7 @@ int detect_launch(const Modulation& mod, const float2* grid, const float2* est, 
   const int64_t share = static_cast<int64_t>((words + segs - 1) / segs) * n * mod.bps;
   const int64_t want = 4 * ((share + 127) / 128 + 1);
   const int bits_words = want * NT * 4 <= 48 * 1024 ? static_cast<int>(want) : 0;
-  const DemapBounds& bounds = bounds_of(mod);
+  const DemapBounds& bounds = demap_bounds_of(mod);
   if (segs > 1)
     hipLaunchKernelGGL(zero_counts_kernel, dim3(static_cast<unsigned>((num_drops + 255) / 256)), dim3(256), 0, stream, errors,
                        num_drops);

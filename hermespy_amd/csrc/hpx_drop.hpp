@@ -571,7 +571,7 @@ __device__ __forceinline__ void drop_body(ConstArgs* ap, const int64_t local_dro
             }
             if (m + 1 >= 0) {
               const float2 h1 = taylor_eval(
-                  coef + (p * a.nb + static_cast<int>(tb.block_of(m + 1))) * kTaylorCoeffs, tb.offset(m + 1));
+                  coef0 + (p * a.nb + static_cast<int>(tb.block_of(m + 1))) * kTaylorCoeffs, tb.offset(m + 1));
 #pragma unroll
               for (int t = 0; t < NT; ++t) z1[t] = cfma(h1, xc[t * a.xs + 1], z1[t]);
             }

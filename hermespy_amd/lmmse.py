@@ -112,7 +112,19 @@ def lmmse_filters(cfg: LinkConfig, snr_db) -> np.ndarray:
 
 class RowSets(list):
     """Device lists of LS rows per SNR point (or None), each row in at most one of them: what
-    :meth:`LMMSEChannelEstimation.rows_by_set` returns, and what one launch can serve at once."""
+    :meth:`LMMSEChannelEstimation.rows_by_set` returns, and what one launch can serve at once while it
+    holds the lists it was made of."""
+
+    def __init__(self, lists=()) -> None:
+        super().__init__(lists)
+        self._made_of = tuple(self)
+
+    @property
+    def disjoint(self) -> bool:
+        """False once a list was replaced, added or taken out: rows may then be in two sets."""
+
+        made_of = getattr(self, "_made_of", ())
+        return len(self) == len(made_of) and all(a is b for a, b in zip(self, made_of))
 
 
 class LMMSEChannelEstimation:
@@ -151,7 +163,7 @@ class LMMSEChannelEstimation:
         if rows_by_set is None:
             rows_by_set = self.rows_by_set(snr_index)
         lib, st = _lib.load(), _lib.stream_handle()
-        if isinstance(rows_by_set, RowSets) and len(rows_by_set) <= self.filters.shape[0]:
+        if isinstance(rows_by_set, RowSets) and rows_by_set.disjoint and len(rows_by_set) <= self.filters.shape[0]:
             lists = (ctypes.c_void_p * len(rows_by_set))(*[_lib.ptr(r) for r in rows_by_set])
             counts = (ctypes.c_int32 * len(rows_by_set))(*[0 if r is None else int(r.numel()) for r in rows_by_set])
             _lib.check(lib.hpx_lmmse_apply_sets(_lib.ptr(ls), c.num_tx, num_drops * c.num_rx, self.num_pilots,
@@ -171,9 +183,9 @@ class LMMSEChannelEstimation:
 
         snr_index = np.asarray(snr_index)
         nr = self.cfg.num_rx
-        out = RowSets()
+        out = []
         for s in range(self.snr_db.size):
             drops = np.flatnonzero(snr_index == s)
             rows = (drops[:, None] * nr + np.arange(nr)[None, :]).reshape(-1).astype(np.int32)
             out.append(torch.as_tensor(rows, device=self.device) if rows.size else None)
-        return out
+        return RowSets(out)

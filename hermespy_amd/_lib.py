@@ -112,12 +112,14 @@ class HpxMassiveWork(ctypes.Structure):
     _fields_ = [(name, c_vp) for name in ("spatial", "coef", "abar", "det_v", "det_a", "det_l", "z", "grid", "csi")]
 
 
-# name -> (restype, argtypes)
 class HpxAdamTensor(ctypes.Structure):
+    """Mirror of ``hpx_adam_tensor`` (device pointers)."""
+
     _fields_ = [("param", c_vp), ("grad", c_vp), ("m1", c_vp), ("m2", c_vp), ("weight", c_vp),
                 ("weight_transposed", c_vp), ("n", c_i64), ("taps", ctypes.c_int32), ("cin", ctypes.c_int32)]
 
 
+# name -> (restype, argtypes)
 SIGNATURES = {
     "hpx_abi_version": (c_int, []),
     "hpx_last_error": (c_int, [ctypes.c_char_p, ctypes.c_size_t]),

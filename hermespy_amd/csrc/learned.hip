@@ -664,8 +664,8 @@ __global__ void __launch_bounds__(256) weight_copies_kernel(const float* __restr
 // wavefront owns whole samples.  Rows of 64 channels are stored with their 16-byte pieces permuted by
 // row (piece ^ (row & 7)), free of bank conflicts without padding: 44 KB for four samples, three workgroups
 // per CU.  All sums keep the order of the layer-by-layer convolutions and so round to the same bfloat16.
-// 16384 samples of 224 output channels on MI355X: 647 -> 481 us (635 TFLOP/s; the matrix cores are busy
-// for 30 % of it and the VALU, with tanhf 28 of some 33 instructions per hidden value, for 50 %); eight
+// 16384 samples of 224 output channels on MI355X: 647 -> 484 us (630 TFLOP/s; the VALU, with tanhf 28 of
+// some 33 instructions per hidden value, is busy for 65 % of it and the matrix cores for 31 %); eight
 // samples a workgroup 495 us, one sample two wavefronts 527 us.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4n __attribute__((ext_vector_type(4)));

@@ -11,9 +11,10 @@ the DC roll, uniformly sampled by a stream's comb pilots), 64 hidden channels,
 GELU (tanh form), plus a linear 17-tap skip convolution from the input to the
 output: about 146k parameters.  Weights and activations are bfloat16,
 products accumulate in float32 on the MFMA units (``hpx_conv1d_forward``);
-training runs on the device with hand-written kernels: backward-data as the
-forward convolution with transposed, flipped weights, float32 weight
-gradients, batch-NMSE loss and Adam, on drops the fused simulator generates
+training runs on the device with hand-written kernels: one launch forward through
+all layers and one backward-data (the forward convolution with transposed, flipped
+weights), the same bits as the layer-by-layer entry points, float32 weight gradients
+(float32 MFMA, sums in the order of those entry points), batch-NMSE loss and Adam, on drops the fused simulator generates
 (``hpx_run_batch_frames`` exports of the received grid and the ideal CSI).
 
 It replaces the interpolation step of ``OrthogonalLeastSquaresChannelEstimation``
@@ -169,8 +170,8 @@ class ConvNetEstimator:
         return out
 
     def estimate(self, ls: torch.Tensor, noise_power: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-        """Channel estimates [num_tx][drops][num_rx][words * N] from LS values (layer by layer, the
-        training path's arithmetic)."""
+        """Channel estimates [num_tx][drops][num_rx][words * N] from LS values, layer by layer: the
+        bits of the training step's fused forward pass."""
 
         c = self.cfg
         num_tx, drops, num_rx, _ = ls.shape

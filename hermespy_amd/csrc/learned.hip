@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256) wgrad_kernel(const uint16_t* __restrict__
 
 // The same partial sums, bit for bit, on the float32 matrix cores.  A K = 1 MFMA adds one product to every
 // accumulator with one rounding, so a chain of them over the chunk's positions is the chain of fmas above (a
-// bf16 MFMA, three times as fast here, sums 16 products in an order of its own; Adam carries that into the
+// bf16 MFMA, nearly five times as fast here, sums 16 products in an order of its own; Adam carries that into the
 // weights, activations round to other bfloat16 values, and the losses that follow leave the tenth digit).
 // v_mfma_f32_16x16x1_4b makes four 16 x 16 blocks at once: a wavefront owns four blocks (16 output channels by 16
 // (tap, ci) columns), the blocks of a workgroup's co group numbered channels first, so any four share an
